@@ -39,7 +39,8 @@
 extern "C" void* mcx_push_errjmp(void* jb);
 extern "C" void mcx_pop_errjmp(void* old);
 void mcx_check_supported(const Config* cfg);
-size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lblock, int* reflect, size_t boxbytes);
+size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lblock, int* reflect, size_t boxbytes,
+                        int pencil);
 
 #define MCX_BATCH_MAXBUF 16
 #define MCX_BATCH_MAXBLOCK ((size_t)MCX_BATCH_BLOCK_MAX)
@@ -183,7 +184,7 @@ static size_t batch_params(MCXBatch* b, size_t lblock, size_t boxbytes) {
         Config* cfg = b->cfg[i];
         MCXKParam& g = b->prm[i];
         int reflect = 0;
-        size_t s = mcx_kparam_setup(cfg, &g, lblock, lblock, &reflect, boxbytes);
+        size_t s = mcx_kparam_setup(cfg, &g, lblock, lblock, &reflect, boxbytes, 0);
         shmem = s > shmem ? s : shmem;
         b->reflect |= reflect;
         g.nrep = 1;
@@ -438,7 +439,7 @@ static void batch_create_impl(MCXBatch* b, Config** cfgs, unsigned int n, MCXBat
         Config* cfg = b->cfg[i];
         MCXKParam g;
         int reflect;
-        (void)mcx_kparam_setup(cfg, &g, 64, 64, &reflect, 0);
+        (void)mcx_kparam_setup(cfg, &g, 64, 64, &reflect, 0, 0);
         b->fieldoff[i + 1] = b->fieldoff[i] + g.fieldlen;
         maxlen = g.fieldlen > maxlen ? g.fieldlen : maxlen;
         nvoxall += g.nvox;

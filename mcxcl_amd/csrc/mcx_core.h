@@ -19,6 +19,8 @@
    for the general path with both, which would spill 21. */
 #define MCX_MAX_BLOCK 256
 #define MCX_FAST_SIMPLE_BLOCK 1024
+/* waves per SIMD the fast kernels are built for (amdgpu_waves_per_eu caps them) */
+#define MCX_FAST_WAVES 4
 #define MCX_FAST_BLOCK 1024
 #define MCX_FAST_DETREF_BLOCK 768
 #define MCX_FAST_BOUND(SAVEDET, REFLECT, SIMPLE) \
@@ -65,7 +67,7 @@ struct MCXKParam {
     uint32_t npattern;            /* patterns sharing each photon (a pattern source with srcnum > 1), else 1;
                                      their slots interleave after the voxel: (vox + gate*nvox)*npattern + k */
     uint32_t nangle;              /* entries of the launch polar-angle table (0: none) */
-    uint32_t pplen;               /* floats of per-lane LDS scratch (records, tallies, w0, source id,
+    uint32_t pplen;               /* floats of per-lane LDS scratch (records, w0, source id,
                                      pattern weights, the RF replay phase) */
     uint32_t imoff;               /* complex outputs (RF replay, RF forward): offset of the imaginary half
                                      (0: real output) */

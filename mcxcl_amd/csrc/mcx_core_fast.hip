@@ -37,8 +37,9 @@ extern "C" hipError_t mcx_launch_fast(const MCXKParam* prm, int nblock, int nthr
 }
 
 /* Resident workgroups per CU of a kernel from its own register and LDS use and
-   gfx950's per-CU resources: 4 SIMDs, each holding at most 8 waves and 512
-   VGPRs per lane allocated in granules of 8, and the device's LDS per CU in
+   gfx950's per-CU resources: 4 SIMDs, each holding at most MCX_FAST_WAVES waves
+   (the kernels' own cap; the hardware's is 8) and 512 VGPRs per lane allocated in
+   granules of 8, and the device's LDS per CU in
    512-byte granules per workgroup.  A workgroup spreads its waves over the 4
    SIMDs.  (The runtime's occupancy query has returned half of this count on
    some MI355X hosts for the same code object, ruling out 1024-lane workgroups
@@ -56,7 +57,7 @@ static int gfx950_occupancy(const void* kernel, int nthreadblock, size_t shmem) 
     const int waves = (nthreadblock + 63) / 64;
     const int perSimd = (waves + 3) / 4;
     const int vgpr = ((a.numRegs > 0 ? a.numRegs : 1) + 7) & ~7;
-    const int simdWaves = (512 / vgpr) < 8 ? (512 / vgpr) : 8;
+    const int simdWaves = (512 / vgpr) < MCX_FAST_WAVES ? (512 / vgpr) : MCX_FAST_WAVES;
     const int byRegs = simdWaves / perSimd;
     const size_t lds = (shmem + a.sharedSizeBytes + 511) & ~(size_t)511;
     const int byLds = lds ? (int)((size_t)ldscu / lds) : byRegs;

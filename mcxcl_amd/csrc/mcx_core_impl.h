@@ -140,6 +140,32 @@ __device__ __forceinline__ float kacos(float x) {
 }
 #endif
 
+/* keeps a value computed in its register where it stands: the compiler otherwise
+   sinks state updates into the later branches that use them and copies every
+   variant of the state at each join */
+#define K_PIN(x) asm("" : "+v"(x))
+
+/* The parameters again, for code that runs rarely: loads through this reference
+   cannot be hoisted into the kernel's prologue, so they hold no scalar registers
+   across the step loop (those that did not fit there were spilled to vector
+   lanes, one v_readlane_b32 per use). */
+typedef const __attribute__((address_space(4))) MCXKParam* KParamPtr;
+__device__ __forceinline__ const MCXKParam& cold(KParamPtr p) {
+    asm("" : "+s"(p));
+    return *(const MCXKParam*)p;
+}
+
+/* Accesses through pointers that come out of memory (the batched launch's parameter
+   blocks, cold()) would be flat ones; these name the global address space. */
+#define K_GLOBAL __attribute__((address_space(1)))
+__device__ __forceinline__ uint32_t media_at(const MCXKParam& g, size_t i) {
+    return ((const K_GLOBAL uint32_t*)g.media)[i];
+}
+
+__device__ __forceinline__ void grid_add(const MCXKParam& g, size_t i, double val) {
+    __builtin_amdgcn_global_atomic_fadd_f64((K_GLOBAL double*)g.field + i, val);
+}
+
 /* sin(acos(x)) for |x| <= 1.  Parity mode evaluates it as the reference writes
    it; fast mode uses the identity sqrt(1 - x^2). */
 __device__ __forceinline__ float ksin_acos(float x) {
@@ -162,14 +188,19 @@ typedef float BoxCell;
 /* ---------------- RNG: xorshift128+ (src/mcx_core.cl:684-698) ---------------- */
 struct Rng {
     uint64_t s0, s1;
+    /* in 32-bit halves: a 64-bit shift is two to four instructions' worth of issue,
+       v_alignbit_b32 and the three-input v_bitop3_b32 (0x96: xor) one each */
     __device__ __forceinline__ float next() {
-        uint64_t x = s0;
-        const uint64_t y = s1;
-        s0 = y;
-        x ^= x << 23;
-        s1 = x ^ y ^ (x >> 18) ^ (y >> 5);
-        uint32_t lo = (uint32_t)(s1 + y);
-        return __uint_as_float(0x3F800000u | (lo >> 9)) - 1.0f;
+        uint32_t xl = (uint32_t)s0, xh = (uint32_t)(s0 >> 32);
+        const uint32_t yl = (uint32_t)s1, yh = (uint32_t)(s1 >> 32);
+        s0 = s1;
+        xh ^= __builtin_amdgcn_alignbit(xh, xl, 9);
+        xl ^= xl << 23;
+        const uint32_t zl = __builtin_amdgcn_bitop3_b32(xl, yl, __builtin_amdgcn_alignbit(xh, xl, 18), 0x96) ^
+                            __builtin_amdgcn_alignbit(yh, yl, 5);
+        const uint32_t zh = __builtin_amdgcn_bitop3_b32(xh, yh, xh >> 18, 0x96) ^ (yh >> 5);
+        s1 = (uint64_t)zh << 32 | zl;
+        return __uint_as_float(__builtin_amdgcn_alignbit(0x7Fu, zl + yl, 9)) - 1.0f;
     }
     __device__ __forceinline__ float scatlen() {
         return -klog(next() + K_EPS);
@@ -181,7 +212,7 @@ __device__ __forceinline__ int to_short(int v) {
 }
 
 __device__ __forceinline__ bool inside(const MCXKParam& g, int x, int y, int z) {
-    return (uint32_t)(x & 0xFFFF) < g.dimx && (uint32_t)(y & 0xFFFF) < g.dimy && (uint32_t)(z & 0xFFFF) < g.dimz;
+    return ((uint32_t)(x & 0xFFFF) < g.dimx) & ((uint32_t)(y & 0xFFFF) < g.dimy) & ((uint32_t)(z & 0xFFFF) < g.dimz);
 }
 
 __device__ __forceinline__ float nextafter_ref(float a, int dir) {
@@ -299,6 +330,7 @@ struct Photon {
     int fx, fy, fz, fw;          /* voxel index (short semantics) and hit face */
     uint32_t idx1d, mediaid;
     float w0, Lmove;
+    float esc, tot;              /* the lane's escaped and launched weight */
     /* split voxel (svmc, src/mcx_core.cl:594-598): the interface plane n.x = pd of
        the current voxel, its normal pointing away from the photon's side, as
        {nx, ny, nz, pd} in the lane's scratch at svoff (sn points there in svmc
@@ -310,6 +342,7 @@ struct Photon {
 };
 
 struct Shared {
+    KParamPtr kp;                /* the run's parameters, for cold() */
     float4* prop;                /* medium table */
     float* invcdf;
     BoxCell* box;                /* privatised deposit box (box_cells) */
@@ -329,42 +362,38 @@ struct DepCache {
     double v0, v1;
 };
 
-__device__ __forceinline__ void depcache_add(const MCXKParam& g, const Shared& sh, DepCache& c, uint32_t addr,
-        float val) {
-    if (addr == c.a0) {
-        c.v0 += (double)val;
-    } else if (addr == c.a1) {
-        c.a1 = c.a0;
-        c.a0 = addr;
-        double t = c.v1 + (double)val;
-        c.v1 = c.v0;
-        c.v0 = t;
-    } else {
-        if (c.a1 != 0xFFFFFFFFu) {
-            atomicAdd(g.field + sh.repoff + c.a1, c.v1);
-        }
+/* adds val at addr; returns whether an entry fell out, in out_a and out_v */
+__device__ __forceinline__ bool depcache_add(DepCache& c, uint32_t addr, float val, uint32_t& out_a, double& out_v) {
+    /* selects, not three branches: a wave's lanes take all of them, and every branch
+       would copy the entries at its join */
+    const bool h0 = addr == c.a0, h1 = addr == c.a1;
 
-        c.a1 = c.a0;
-        c.v1 = c.v0;
-        c.a0 = addr;
-        c.v0 = (double)val;
-    }
+    const bool evict = !(h0 | h1) & (c.a1 != 0xFFFFFFFFu);
+    out_a = c.a1;
+    out_v = c.v1;
+
+    const double sum = (h0 ? c.v0 : (h1 ? c.v1 : 0.0)) + (double)val;
+    c.a1 = h0 ? c.a1 : c.a0;
+    c.v1 = h0 ? c.v1 : c.v0;
+    c.a0 = addr;
+    c.v0 = sum;
+    return evict;
 }
 
 __device__ __forceinline__ void depcache_flush(const MCXKParam& g, const Shared& sh, DepCache& c) {
     if (c.a0 != 0xFFFFFFFFu) {
-        atomicAdd(g.field + sh.repoff + c.a0, c.v0);
+        grid_add(g, sh.repoff + c.a0, c.v0);
     }
 
     if (c.a1 != 0xFFFFFFFFu) {
-        atomicAdd(g.field + sh.repoff + c.a1, c.v1);
+        grid_add(g, sh.repoff + c.a1, c.v1);
     }
 
     c.a0 = c.a1 = 0xFFFFFFFFu;
 }
 
-/* voxel-exit deposit: LDS box when the voxel and gate fall inside it, else the
-   lane's write-combining buffer in front of the global grid.
+/* Voxel-exit deposits go to the LDS box when the voxel and gate fall inside it, else
+   to the lane's write-combining buffer in front of the global grid.
 
    A float32 box cell (fast build) keeps its magnitude below K_BOX_MOVE: the
    lane whose add finds the cell above it moves K_BOX_MOVE (exactly
@@ -374,27 +403,25 @@ __device__ __forceinline__ void depcache_flush(const MCXKParam& g, const Shared&
    many photons a workgroup runs, and the moved amount is exact, so nothing is
    lost or counted twice when several lanes move at once. */
 #define K_BOX_MOVE 1024.f
-__device__ __forceinline__ void deposit_voxel(const MCXKParam& g, const Shared& sh, DepCache& c, int ox, int oy,
-        int oz, uint32_t idx1d, int tshift, float val) {
-    uint32_t dx = (uint32_t)(ox - (int)g.box_x0), dy = (uint32_t)(oy - (int)g.box_y0);
-    uint32_t dz = (uint32_t)(oz - (int)g.box_z0);
 
-    if (dx < g.box_nx && dy < g.box_ny && dz < g.box_nz && (uint32_t)tshift < g.box_ng) {
-        BoxCell* cell = sh.box + (((uint32_t)tshift * g.box_nz + dz) * g.box_ny + dy) * g.box_nx + dx;
-#if MCX_PARITY
-        atomicAdd(cell, (BoxCell)val);
-#else
-        const float old = atomicAdd(cell, val);
+/* a * b + c of factors below 2^24, at the full rate (the compiler prefers the
+   quarter-rate v_mad_u64_u32) */
+__device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) {
+    uint32_t r;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    return r;
+}
 
-        if (fabsf(old) > K_BOX_MOVE) {
-            const float mv = old > 0.f ? K_BOX_MOVE : -K_BOX_MOVE;
-            atomicAdd(cell, -mv);
-            atomicAdd(g.field + sh.repoff + idx1d + (uint32_t)tshift * g.nvox, (double)mv);
-        }
-#endif
-    } else {
-        depcache_add(g, sh, c, idx1d + (uint32_t)tshift * g.nvox, val);
-    }
+/* offset of a box cell; every factor is below 2^24 (the box holds at most 160 KB) */
+__device__ __forceinline__ uint32_t box_offset(const MCXKParam& g, uint32_t gate, uint32_t dx, uint32_t dy, uint32_t dz) {
+    return mad24(mad24(mad24(gate, g.box_nz, dz), g.box_ny, dy), g.box_nx, dx);
+}
+
+/* the move of an overfull cell: idx the cell's place in the replica of the grid */
+__device__ __forceinline__ void box_move(const MCXKParam& g, const Shared& sh, BoxCell* cell, float old, uint32_t idx) {
+    const float mv = old > 0.f ? K_BOX_MOVE : -K_BOX_MOVE;
+    atomicAdd(cell, (BoxCell)(-mv));
+    grid_add(g, sh.repoff + idx, (double)mv);
 }
 
 /* binary16 bit pattern (sign bit clear) to float, exactly, subnormals included */
@@ -471,7 +498,7 @@ __device__ __forceinline__ float4 svmc_prop(const MCXKParam& g, const float4* t,
         return t[0];
     }
 
-    const uint32_t lo = g.media[idx1d + g.nvox];           /* bytes c0..c3: nz, ny, nx, pz */
+    const uint32_t lo = media_at(g, idx1d + g.nvox);           /* bytes c0..c3: nz, ny, nx, pz */
     const uint32_t hi = mediaid & K_MED_MASK;                /* bytes c4..c7: py, px, upper, lower */
     const uint32_t c6 = (hi >> 16) & 0xFFu, c7 = hi >> 24;
     uint32_t sv = c7 | (c6 << 8);
@@ -595,21 +622,64 @@ __device__ __forceinline__ int svmc_reflect(float n1, float4& v, Photon& s, cons
     return 0;
 }
 
+/* what a run uses, as bits (see transport_lane) */
+enum {kfGscatter = 1u << 0, kfPerVoxel = 1u << 1, kfPacked = 1u << 2, kfSvmc = 1u << 3, kfRf = 1u << 4,
+      kfSave = 1u << 5, kfFlux = 1u << 6, kfReflect = 1u << 7, kfPathTally = 1u << 8, kfPatterns = 1u << 9,
+      kfSlots = 1u << 10, kfMoveOnly = 1u << 11, kfPhase = 1u << 12, kf2D = 1u << 13, kfPol = 1u << 14,
+      kfScatDeposit = 1u << 15, kfTraj = 1u << 16, kfCountTally = 1u << 17, kfMomTally = 1u << 18, kfRfReplay = 1u << 19
+     };
+
+__device__ __forceinline__ uint32_t features(const MCXKParam& g) {
+    const uint32_t replay = g.seed == K_SEED_FROM_FILE;
+    uint32_t w = 0;
+    /* the scattering count is a float that stops at 2^24: a larger gscatter is never reached */
+    w |= g.gscatter < (1u << 25) ? kfGscatter : 0u;
+    w |= g.muamus ? kfPerVoxel : 0u;
+    w |= (g.mediaformat > 4 && !g.svmc) ? kfPacked : 0u;
+    w |= g.svmc ? kfSvmc : 0u;
+    w |= g.rfforward ? kfRf : 0u;
+    w |= g.save2pt ? kfSave : 0u;
+    w |= (g.outputtype == kFlux || g.outputtype == kFluence) ? kfFlux : 0u;
+    w |= g.doreflect ? kfReflect : 0u;
+    w |= (g.savedetflag & 4u) ? kfPathTally : 0u;
+    w |= (g.savedetflag & 2u) ? kfCountTally : 0u;
+    w |= (g.savedetflag & 8u) ? kfMomTally : 0u;
+    w |= g.npattern > 1 ? kfPatterns : 0u;
+    w |= (g.extrasrclen && g.srcid < 0) ? kfSlots : 0u;
+    w |= g.moveonly ? kfMoveOnly : 0u;
+    w |= g.nphase > 2 ? kfPhase : 0u;
+    w |= g.is2d ? kf2D : 0u;
+    w |= g.maxpolmedia ? kfPol : 0u;
+    w |= (g.outputtype == kWP || g.outputtype == kDCS || g.outputtype == kWPTOF || (replay && g.outputtype == kRFmus)) ?
+         kfScatDeposit : 0u;
+    w |= g.savetraj ? kfTraj : 0u;
+    w |= (replay && g.outputtype == kRF && g.omega > 0.f) ? kfRfReplay : 0u;
+    return w;
+}
+
 /* the properties of the photon's voxel: label table, per-voxel mua/mus
    replacing the label's, or (full general path) a packed media word */
 template <bool FULL = false>
-__device__ __forceinline__ float4 getprop(const MCXKParam& g, const Shared& sh, uint32_t mediaid, uint32_t idx1d) {
-    if (FULL && g.mediaformat > 4) {
+__device__ __forceinline__ float4 getprop(const MCXKParam& g, const Shared& sh, uint32_t mediaid, uint32_t idx1d,
+        uint32_t ft) {
+    if (FULL && (ft & kfPacked)) {
         return media_word_prop(g.mediaformat, sh.prop, mediaid);
     }
 
     float4 p = sh.prop[mediaid & K_MED_MASK];
 
-    /* per-voxel absorption and scattering: g and n stay those of the label */
-    if (g.muamus && (mediaid & K_MED_MASK)) {
-        float2 m = g.muamus[idx1d];
-        p.x = m.x;
-        p.y = m.y;
+    /* per-voxel absorption and scattering: g and n stay those of the label.  The
+       label's own values are read first, whatever follows: a select between the LDS
+       table and the array would become one flat load, which waits on both counters. */
+    if (ft & kfPerVoxel) {
+        K_PIN(p.x);
+        K_PIN(p.y);
+
+        if ((mediaid & K_MED_MASK) && idx1d < g.nvox) {
+            const K_GLOBAL float* m = (const K_GLOBAL float*)g.muamus + 2 * (size_t)idx1d;
+            p.x = m[0];
+            p.y = m[1];
+        }
     }
 
     return p;
@@ -630,7 +700,7 @@ static __device__ int skipvoid(const MCXKParam& g, Photon& s) {
         if (inside(g, s.fx, s.fy, s.fz)) {
             idx1d = s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx;
 
-            if (g.media[idx1d] & K_MED_MASK) {
+            if (media_at(g, idx1d) & K_MED_MASK) {
                 p.x -= v.x;
                 p.y -= v.y;
                 p.z -= v.z;
@@ -641,7 +711,7 @@ static __device__ int skipvoid(const MCXKParam& g, Photon& s) {
                 idx1d = s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx;
                 count = 0;
 
-                while (!inside(g, s.fx, s.fy, s.fz) || !(g.media[idx1d] & K_MED_MASK)) {
+                while (!inside(g, s.fx, s.fy, s.fz) || !(media_at(g, idx1d) & K_MED_MASK)) {
                     int face;
                     float dist = hitgrid(p, v, s.fx, s.fy, s.fz, &face);
                     s.fw = face;
@@ -680,10 +750,10 @@ static __device__ int skipvoid(const MCXKParam& g, Photon& s) {
                 float nin;
 
                 if (FULL && g.svmc) {
-                    nin = svmc_prop(g, g.prop, g.media[idx1d], (uint32_t)idx1d, p, s.fx, s.fy, s.fz, s).w;
+                    nin = svmc_prop(g, g.prop, media_at(g, idx1d), (uint32_t)idx1d, p, s.fx, s.fy, s.fz, s).w;
                 } else {
-                    nin = (FULL && g.mediaformat > 4) ? media_word_prop(g.mediaformat, g.prop, g.media[idx1d]).w :
-                          g.prop[g.media[idx1d] & K_MED_MASK].w;
+                    nin = (FULL && g.mediaformat > 4) ? media_word_prop(g.mediaformat, g.prop, media_at(g, idx1d)).w :
+                          g.prop[media_at(g, idx1d) & K_MED_MASK].w;
                 }
 
                 if (g.isspecular && nin != g.prop[0].w) {
@@ -829,7 +899,7 @@ __device__ __forceinline__ int gate_of(const MCXKParam& g, float t) {
 
 /* global deposit into this lane's accumulator replica */
 __device__ __forceinline__ void deposit(const MCXKParam& g, size_t repoff, uint32_t addr, float val) {
-    atomicAdd(g.field + repoff + addr, (double)val);
+    grid_add(g, repoff + addr, (double)val);
 }
 
 /* the imaginary half of an RF forward deposit: into the box's second set of
@@ -842,16 +912,14 @@ __device__ __forceinline__ void deposit_voxel_im(const MCXKParam& g, const Share
     const uint32_t addr = idx1d + (uint32_t)tshift * g.nvox + g.imoff;
 
     if (g.box_imgate && dx < g.box_nx && dy < g.box_ny && dz < g.box_nz && (uint32_t)tshift < g.box_ng) {
-        BoxCell* cell = sh.box + ((((uint32_t)tshift + g.box_ng) * g.box_nz + dz) * g.box_ny + dy) * g.box_nx + dx;
+        BoxCell* cell = sh.box + box_offset(g, (uint32_t)tshift + g.box_ng, dx, dy, dz);
 #if MCX_PARITY
         atomicAdd(cell, (BoxCell)val);
 #else
         const float old = atomicAdd(cell, val);
 
         if (fabsf(old) > K_BOX_MOVE) {
-            const float mv = old > 0.f ? K_BOX_MOVE : -K_BOX_MOVE;
-            atomicAdd(cell, -mv);
-            atomicAdd(g.field + sh.repoff + addr, (double)mv);
+            box_move(g, sh, cell, old, addr);
         }
 #endif
     } else {
@@ -860,7 +928,7 @@ __device__ __forceinline__ void deposit_voxel_im(const MCXKParam& g, const Share
 }
 
 /* src/mcx_core.cl:838-926 */
-template <bool SAVEDET, bool FULL>
+template <bool SAVEDET, bool SIMPLE, bool FULL>
 __device__ void save_detected(const MCXKParam& g, const Shared& sh, const Photon& s, uint32_t isdet) {
     int detid = 0;
 
@@ -906,7 +974,7 @@ __device__ void save_detected(const MCXKParam& g, const Shared& sh, const Photon
     uint32_t k = 0;
 
     if (g.savedetflag & 0x1) {
-        if (g.extrasrclen && g.srcid <= 0) {
+        if (!SIMPLE && g.extrasrclen && g.srcid <= 0) {
             detid |= ((int)sh.pp[g.w0offset - 1]) << 16;
         }
 
@@ -930,7 +998,7 @@ __device__ void save_detected(const MCXKParam& g, const Shared& sh, const Photon
     }
 
     if ((g.savedetflag >> 6) & 1) {
-        rec[k++] = sh.pp[g.w0offset - 2];
+        rec[k++] = SIMPLE ? g.srcpos.w : sh.pp[g.w0offset - 2];
     }
 
     if (FULL && ((g.savedetflag >> 7) & 1)) {
@@ -948,12 +1016,12 @@ __device__ void save_detected(const MCXKParam& g, const Shared& sh, const Photon
 __device__ __forceinline__ void pattern_weights(const MCXKParam& g, float* ppl, float4& p, int pix, float srcw) {
     if (g.npattern <= 1) {
         p.w = srcw * g.srcpattern[pix];
-        ppl[4] = p.w;
+        ppl[2] = p.w;
     } else {
-        ppl[2] = __uint_as_float((uint32_t)pix);
+        ppl[0] = __uint_as_float((uint32_t)pix);
 
         for (uint32_t i = 0; i < g.npattern; i++) {
-            ppl[4 + i] = g.srcpattern[(size_t)pix * g.npattern + i];
+            ppl[2 + i] = g.srcpattern[(size_t)pix * g.npattern + i];
         }
 
         p.w = 1.f;
@@ -964,7 +1032,11 @@ __device__ __forceinline__ void pattern_weights(const MCXKParam& g, float* ppl, 
    Returns 0 on a launch, 1 when the lane's photon budget is used up, -1 when
    no launch succeeded within maxvoidstep attempts. */
 template <bool SAVEDET, bool SIMPLE, bool FULL>
-__device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rng& rng, int idx, uint32_t isdet) {
+__device__ __forceinline__ int launch_photon(const MCXKParam& gk, const Shared& sh, Photon& s, Rng& rng, int idx, uint32_t isdet,
+        uint32_t ft) {
+    /* the pencil beam's launch reads few parameters and runs in a sixth of a wave's
+       steps: those stay in registers */
+    const MCXKParam& g = SIMPLE ? gk : cold(sh.kp);
     float* pp = sh.pp;
     const uint32_t pd = g.partialdata;
     float4& p = s.p;
@@ -973,7 +1045,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
     s.w0 = 1.f;
     s.Lmove = -1.f;
 
-    if (SAVEDET && g.savedet == K_FILL_MAXDET && __hip_atomic_load(g.detcount, __ATOMIC_RELAXED,
+    if (SAVEDET && !SIMPLE && g.savedet == K_FILL_MAXDET && __hip_atomic_load(g.detcount, __ATOMIC_RELAXED,
             __HIP_MEMORY_SCOPE_AGENT) >= g.maxdetphoton) {
         /* fill-max mode (src/mcx_core.cl:1484-1489): the lane stops once the
            detected-photon buffer is full */
@@ -981,7 +1053,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
     }
 
     if (fabsf(p.w) >= 0.f) {
-        pp[pd] += p.w;
+        s.esc += p.w;
 
         if (FULL && g.savetraj) {
             save_traj(g, p, photon_index(g, idx, f.w), pp[g.w0offset - 1], pp + g.stokesoff);
@@ -1030,7 +1102,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
 
         if (SAVEDET && (isdet & K_DET_MASK) == K_DET_MASK &&
                 (s.mediaid == 0 || (FULL && g.svmc && K_SV_CURLABEL(s.sv) == 0)) && g.issaveref < 2) {
-            save_detected<SAVEDET, FULL>(g, sh, s, isdet);
+            save_detected<SAVEDET, SIMPLE, FULL>(cold(sh.kp), sh, s, isdet);
         }
     }
 
@@ -1067,10 +1139,9 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
         s.fy = to_short((int)floorf(p.y));
         s.fz = to_short((int)floorf(p.z));
         f.w += 1.f;
-        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d);
-        pp[pd + 1] += p.w;
+        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+        s.tot += p.w;
         s.w0 = p.w;
-        pp[pd + 2] = (g.srcnum > 1) ? pp[pd + 2] : p.w;
         v.w = K_EPS;
         s.Lmove = 0.f;
         return 0;
@@ -1114,7 +1185,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
         rng.next();
     }
 
-    float* ppl = pp + pd;
+    float* ppl = pp + pd;       /* launch weight, source id, pattern weights */
 
     do {
         p = lpos;
@@ -1370,7 +1441,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
                 if (p.x < 0.f || p.y < 0.f || p.z < 0.f || p.x >= g.maxidx_x || p.y >= g.maxidx_y || p.z >= g.maxidx_z) {
                     s.mediaid = 0;
                 } else {
-                    s.mediaid = g.media[s.idx1d];
+                    s.mediaid = media_at(g, s.idx1d);
                 }
             }
         }
@@ -1459,7 +1530,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
             if (p.x < 0.f || p.y < 0.f || p.z < 0.f || p.x >= g.maxidx_x || p.y >= g.maxidx_y || p.z >= g.maxidx_z) {
                 s.mediaid = 0;
             } else {
-                s.mediaid = g.media[s.idx1d];
+                s.mediaid = media_at(g, s.idx1d);
             }
         }
 
@@ -1468,7 +1539,7 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
 
             if (id >= 0) {
                 s.idx1d = (uint32_t)id;
-                s.mediaid = g.media[s.idx1d];
+                s.mediaid = media_at(g, s.idx1d);
             }
         }
 
@@ -1484,15 +1555,15 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
 
     f.w += 1.f;
     s.prop = (FULL && g.svmc) ? svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s) :
-             getprop<FULL>(g, sh, s.mediaid, s.idx1d);
+             getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
 
     if (FULL && g.savetraj) {
-        save_traj(g, p, traj_index(g, idx, f.w), ppl[3], pp + g.stokesoff);   /* the source-id slot */
+        save_traj(g, p, traj_index(g, idx, f.w), ppl[1], pp + g.stokesoff);   /* the source-id slot */
     }
 
-    ppl[1] += p.w;
+    s.tot += p.w;
     s.w0 = p.w;
-    ppl[2] = (g.srcnum > 1) ? ppl[2] : p.w;
+    ppl[0] = (g.srcnum > 1) ? ppl[0] : p.w;
     v.w = K_EPS;
     s.Lmove = 0.f;
 
@@ -1501,20 +1572,61 @@ __device__ int launch_photon(const MCXKParam& g, const Shared& sh, Photon& s, Rn
            which reads the next photon's time of flight; here the photon's own) */
         float rs, rc;
         ksincos(g.omega * g.replaytof[photon_index(g, idx, f.w) - 1], &rs, &rc);
-        ppl[4 + g.srcnum] = rc;
-        ppl[5 + g.srcnum] = rs;
+        ppl[2 + g.srcnum] = rc;
+        ppl[3 + g.srcnum] = rs;
     }
 
     return 0;
 }
 
+/* boundary codes of the three faces at index 0 (o = 0) or at the far end (o = 3),
+   one byte each, the default filled in; uniform, so it lives in one scalar register
+   and a photon at a face reads it with a shift instead of a load */
+__device__ __forceinline__ uint32_t bc_codes(const MCXKParam& g, int o) {
+    const uint32_t dflt = g.doreflect ? (uint32_t)kReflect : (uint32_t)kAbsorb;
+    uint32_t w = 0;
+
+    for (int i = 0; i < 3; i++) {
+        const uint32_t c = g.bc[o + i];
+        w |= ((c & 0xFu) ? c : dflt) << (8 * i);
+    }
+
+    return w;
+}
+
+/* the faces whose escaping photons are detected: bit i for face i at index 0, bit
+   3 + i for the far face (bc[6..11]) */
+__device__ __forceinline__ uint32_t bc_detects(const MCXKParam& g) {
+    uint32_t w = 0;
+
+    for (int i = 0; i < 6; i++) {
+        w |= (g.bc[6 + i] ? 1u : 0u) << i;
+    }
+
+    return w;
+}
+
+/* What bounds the step loop: instruction issue of a wave (most steps of a wave take
+   every branch), then the waits for the label and the grid atomic behind it.  So the
+   state is updated in place under selects (K_PIN), a run's options sit in one scalar
+   register (features), boundary codes in another, rare branches share one test, the
+   label and the properties are read only where the voxel changes, and the energy
+   tallies are registers, which leaves their LDS to the deposit box.  Measured against
+   the loop that reloaded label and properties at every step (MI355X, kernel time):
+   packed media, isotropic source, 71x64x53, 3e6 photons 169 -> 113 ms; layered 200^3,
+   1e7 photons 151 -> 122 ms; 60^3 pencil beam, 3e5 photons 7.2 -> 6.0 ms; batch of 16
+   48^3 instances 867 -> 764 ms; the 60^3 sphere at 1e8 photons, which the grid
+   atomics bound, 423 -> 421 ms. */
 /* Transport this lane's photons until its share (fixed map) or its
    workgroup's pool (run-time hand-out) is exhausted.  The photon state starts
    fresh; the RNG, the LDS tables and the lane's scratch come in, and the
    lane's pending grid deposits are flushed before returning. */
 template <bool SAVEDET, bool REFLECT, bool SIMPLE, bool FULL>
-__device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared& sh, Rng& rng, const int idx) {
+__device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared& sh, Rng& rng, const int idx,
+        float& esc, float& tot) {
     Photon s;
+    s.esc = esc;
+    s.tot = tot;
     s.p = make_float4(0.f, 0.f, 0.f, __uint_as_float(0x7FC00000u));
     s.v = make_float4(0.f, 0.f, 0.f, 0.f);
     s.f = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1526,14 +1638,26 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
     s.w0 = 0.f;
     s.Lmove = 0.f;
 
-    uint32_t isdet = 0, mediaidold = 0, idx1dold = 0, launchflag = 0;
+    /* the detector flag in effect: the voxel's own, except after a reflection, where
+       the reference keeps what the step found beyond the face until the photon's next
+       step inside the voxel; detvox is the voxel's own */
+    uint32_t isdet = 0, detvox = 0, launchflag = 0;
     float pathlen = 0.f, n1 = 0.f;
     bool relaunch = true;
-    /* coordinates of the voxel idx1dold names.  After a reflection idx1d is restored
-       while the integer position keeps the reflected face's index for one step, so the
-       previous coordinates are kept across that step. */
-    int ox = 0, oy = 0, oz = 0;
-    bool keepold = false;
+    /* linear index of the integer position.  It is idx1d's except after a reflection,
+       when idx1d is restored while the position keeps the reflected face's index for
+       one step (at a face on the voxel's far side the next voxel's); a deposit then
+       goes by idx1d alone, past the box */
+    uint32_t lin = 0;
+    const uint32_t feat0 = features(g);
+    uint32_t detsrc = 0;
+
+    if (SAVEDET && SIMPLE && __float_as_uint(g.srcparam2.z) < g.nvox) {
+        detsrc = media_at(g, __float_as_uint(g.srcparam2.z)) & K_DET_MASK;
+    }
+
+    const uint32_t bcmin = bc_codes(g, 0), bcmax = bc_codes(g, 3), bcdet = bc_detects(g);
+    const float n0 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sh.prop[0].w)));
     DepCache dcache;
     dcache.a0 = dcache.a1 = 0xFFFFFFFFu;
     dcache.v0 = dcache.v1 = 0.0;
@@ -1558,16 +1682,23 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 
     for (;;) {
         if (relaunch) {
-            if (launch_photon<SAVEDET, SIMPLE, FULL>(g, sh, s, rng, idx, launchflag)) {
+            if (launch_photon<SAVEDET, SIMPLE, FULL>(g, sh, s, rng, idx, launchflag, feat0)) {
                 break;
             }
 
             isdet = s.mediaid & K_DET_MASK;
             s.mediaid &= K_MED_MASK;
-            relaunch = false;
-            keepold = false;
+            n1 = s.prop.w;
 
-            if (FULL && g.rfforward) {
+            if (SAVEDET) {
+                /* a source's own label carries no detector flag: the volume's has it */
+                detvox = SIMPLE ? detsrc : (s.idx1d < g.nvox ? media_at(g, s.idx1d) & K_DET_MASK : 0u);
+            }
+
+            lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+            relaunch = false;
+
+            if (FULL && (feat0 & kfRf)) {
                 rf.wre = sh.pp[g.rfoff] = s.p.w;
                 rf.wim = sh.pp[g.rfoff + 1] = 0.f;
             }
@@ -1576,6 +1707,10 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         float4& p = s.p;
         float4& v = s.v;
         float4& f = s.f;
+        /* one scalar register holds what the run uses; hidden from the compiler at each
+           step, or every test would be hoisted into a register pair of its own */
+        uint32_t ft = feat0;
+        asm("" : "+s"(ft));
 
         if (f.x <= 0.f) {
             f.x = rng.scatlen();
@@ -1583,7 +1718,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
             if (v.w != K_EPS) {
                 float cphi = 1.f, sphi = 0.f, theta = 0.f, stheta, ctheta, tmp0 = 0.f;
 
-                if (FULL && g.maxpolmedia && !g.is2d) {
+                if (FULL && (ft & kfPol) && !(ft & kf2D)) {
                     /* polarised media (src/mcx_core.cl:2454-2468): (theta, phi) by rejection
                        against I(theta, phi) = S11 I + S12 (Q cos 2phi + U sin 2phi) of the
                        medium's table, the forward entry as the bound */
@@ -1641,12 +1776,12 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 #endif
                     ksincos(tmp0, &sphi, &cphi);
                 } else {
-                if (SIMPLE || !g.is2d) {
+                if (SIMPLE || !(ft & kf2D)) {
                     tmp0 = K_TWO_PI * rng.next();
                     ksincos(tmp0, &sphi, &cphi);
                 }
 
-                if (!SIMPLE && g.nphase > 2) {
+                if (!SIMPLE && (ft & kfPhase)) {
                     tmp0 = rng.next() * (float)(g.nphase - 1);
                     theta = tmp0 - (float)((int)tmp0);
                     uint32_t i0 = (uint32_t)tmp0 >= g.nphase ? g.nphase - 1 : (uint32_t)(int)tmp0;
@@ -1655,11 +1790,11 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     stheta = ksin_acos(tmp0);
                     ctheta = tmp0;
 
-                    if (FULL && g.maxpolmedia) {
+                    if (FULL && (ft & kfPol)) {
                         theta = kacos(tmp0);    /* the angle the Stokes update takes (2D polarised runs) */
                     }
                 } else {
-                    tmp0 = (v.w > (float)g.gscatter) ? 0.f : s.prop.z;
+                    tmp0 = ((ft & kfGscatter) && v.w > (float)g.gscatter) ? 0.f : s.prop.z;
 
                     if (fabsf(tmp0) > K_EPS) {
                         tmp0 = kdiv(1.f - s.prop.z * s.prop.z, 1.f - s.prop.z + 2.f * s.prop.z * rng.next());
@@ -1669,7 +1804,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                         stheta = ksin_acos(tmp0);
                         ctheta = tmp0;
 
-                        if (FULL && g.maxpolmedia) {
+                        if (FULL && (ft & kfPol)) {
                             theta = kacos(tmp0);
                         }
                     } else {
@@ -1680,7 +1815,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                         ctheta = 2.f * rng.next() - 1.f;
                         stheta = ksin_acos(ctheta);
 
-                        if (FULL && g.maxpolmedia) {
+                        if (FULL && (ft & kfPol)) {
                             theta = kacos(ctheta);
                         }
 #endif
@@ -1689,15 +1824,15 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                 }
 
                 /* per-medium tallies: a split voxel's current side (src/mcx_core.cl:2502-2540) */
-                const uint32_t tlab = (FULL && g.svmc) ? K_SV_CURLABEL(s.sv) : (s.mediaid & K_MED_MASK);
+                const uint32_t tlab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : (s.mediaid & K_MED_MASK);
 
                 if (SAVEDET && tlab > 0) {
-                    if ((g.savedetflag >> 1) & 1) {
+                    if (ft & kfCountTally) {
                         uint32_t* cnt = (uint32_t*)sh.pp;
                         cnt[tlab - 1]++;
                     }
 
-                    if ((g.savedetflag >> 3) & 1) {
+                    if (ft & kfMomTally) {
                         sh.pp[g.maxmedia * (((g.savedetflag >> 1) & 1) + ((g.savedetflag >> 2) & 1)) + tlab - 1] +=
                             1.f - ctheta;
                     }
@@ -1705,7 +1840,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 
                 const float4 olddir = v;
 
-                if (!SIMPLE && g.is2d) {
+                if (!SIMPLE && (ft & kf2D)) {
                     rotatevector2d(v, (rng.next() > 0.5f ? stheta : -stheta), ctheta, (int)g.is2d);
                 } else {
                     rotatevector(v, stheta, ctheta, sphi, cphi);
@@ -1713,7 +1848,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 
                 v.w += 1.f;
 
-                if (FULL && g.maxpolmedia) {
+                if (FULL && (ft & kfPol)) {
                     /* :2550-2565; in 2D the reference samples by HG with the medium's g and
                        passes the sampled cosine (tmp0) where the azimuth goes */
                     float4 st = stokes_get(g, sh.pp);
@@ -1721,9 +1856,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     stokes_put(g, sh.pp, st);
                 }
 
-                if (!SIMPLE && (g.outputtype == kWP || g.outputtype == kDCS ||
-                                (FULL && (g.outputtype == kWPTOF ||
-                                          (g.seed == K_SEED_FROM_FILE && g.outputtype == kRFmus))))) {
+                if (!SIMPLE && (ft & kfScatDeposit) && (FULL || g.outputtype == kWP || g.outputtype == kDCS)) {
                     /* replay deposits at each scattering site (src/mcx_core.cl:2568-2623):
                        w (WP), (1 - cos theta) w (DCS), tof w (WPTOF), w e^{i omega tof} (RFmus) */
                     uint32_t pid = photon_index(g, idx, f.w) - 1;
@@ -1756,32 +1889,42 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     }
                 }
 
-                if (FULL && g.savetraj) {
+                if (FULL && (ft & kfTraj)) {
                     save_traj(g, p, traj_index(g, idx, f.w), sh.pp[g.w0offset - 1], sh.pp + g.stokesoff);
                 }
             }
 
             v.w = (float)(int)v.w;
 
-            if (FULL && g.svmc) {
+            if (FULL && (ft & kfSvmc)) {
                 testint = true;
             }
         }
 
-        n1 = s.prop.w;
-        /* split voxels: the side is taken again from the position at every step
+        /* s.prop holds the properties of the photon's voxel and n1 its index; split
+           voxels: the side is taken again from the position at every step
            (src/mcx_core.cl:2656-2672) */
-        s.prop = (FULL && g.svmc) ? svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s) :
-                 getprop<FULL>(g, sh, s.mediaid, s.idx1d);
+        if (FULL && (ft & kfSvmc)) {
+            n1 = s.prop.w;
+            s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
+        }
+
         int face;
         f.z = hitgrid(p, v, s.fx, s.fy, s.fz, &face);
-        s.fw = face;
-        float gfac = (v.w + 1.f > (float)g.gscatter ? (1.f - s.prop.z) : 1.f);
+        float gfac = 1.f;
+
+        if (ft & kfGscatter) {
+            gfac = (v.w + 1.f > (float)g.gscatter ? (1.f - s.prop.z) : 1.f);
+            K_PIN(gfac);
+        }
+
         float slen = f.z * s.prop.y * gfac;
-        slen = fminf(slen, f.x);
+        /* the scattering site comes before the face */
+        bool stay = !(slen < f.x);
+        slen = stay ? f.x : slen;
         f.z = kdiv(slen, s.prop.y * gfac);
 
-        if (FULL && g.svmc) {
+        if (FULL && (ft & kfSvmc)) {
             /* the step ends on the voxel's plane when it crosses it (src/mcx_core.cl:2684-2701) */
             hitintf = false;
 
@@ -1791,33 +1934,47 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                 f.z = len;
             }
         }
-        if (!keepold) {
-            ox = s.fx;
-            oy = s.fy;
-            oz = s.fz;
-        }
 
-        keepold = false;
         pathlen += f.z;
         p.x = p.x + f.z * v.x;
         p.y = p.y + f.z * v.y;
         p.z = p.z + f.z * v.z;
+        K_PIN(p.x);
+        K_PIN(p.y);
+        K_PIN(p.z);
 
-        const bool stay = (slen == f.x) || (FULL && hitintf);
+        stay = stay | (FULL && hitintf);
+        float vface = v.z;
+        int lstep = (int)g.dimxy;
+        vface = (face == 1) ? v.y : vface;
+        lstep = (face == 1) ? (int)g.dimx : lstep;
+        vface = (face == 0) ? v.x : vface;
+        lstep = (face == 0) ? 1 : lstep;
+        const int sgn = stay ? 0 : (vface > 0.f ? 1 : -1);
+        const uint32_t lin0 = lin;
+        lin += (uint32_t)(stay ? 0 : (vface > 0.f ? lstep : -lstep));
+        /* the voxel the photon leaves, and the one it is in now */
+        const int cx = s.fx, cy = s.fy, cz = s.fz;
+        s.fx += (face == 0) ? sgn : 0;
+        s.fy += (face == 1) ? sgn : 0;
+        s.fz += (face == 2) ? sgn : 0;
+        K_PIN(s.fx);
+        K_PIN(s.fy);
+        K_PIN(s.fz);
 
-        if (face == 0) {
-            s.fx += stay ? 0 : (v.x > 0.f ? 1 : -1);
+        /* the label is loaded only where the voxel changes, ahead of the arithmetic
+           that does not need it */
+        const bool in = inside(g, s.fx, s.fy, s.fz);
+        const uint32_t oidx = s.idx1d, omed = s.mediaid;
+        s.idx1d = in ? lin : (((s.fx | s.fy | s.fz) < 0) ? K_OUT_MIN : K_OUT_MAX);
+        const bool cross = s.idx1d != oidx;
+        uint32_t lab = 0;
+
+        if (in & cross) {
+            lab = media_at(g, s.idx1d);
         }
 
-        if (face == 1) {
-            s.fy += stay ? 0 : (v.y > 0.f ? 1 : -1);
-        }
-
-        if (face == 2) {
-            s.fz += stay ? 0 : (v.z > 0.f ? 1 : -1);
-        }
-
-        if (FULL && g.rfforward) {
+        if (FULL && (ft & kfRf)) {
             /* RF forward (src/mcx_core.cl:2750-2760): w <- w exp(-(mua + i omega n / c0) ds),
                p.w its magnitude */
             const float att = kexp(-s.prop.x * f.z);
@@ -1835,116 +1992,157 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         f.x -= slen;
         f.y += f.z * s.prop.w * g.oneoverc0;
 
-        if (SAVEDET && ((g.savedetflag >> 2) & 1)) {
-            const uint32_t plab = (FULL && g.svmc) ? K_SV_CURLABEL(s.sv) : (s.mediaid & K_MED_MASK);
+        if (SAVEDET && (ft & kfPathTally)) {
+            const uint32_t plab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : (s.mediaid & K_MED_MASK);
 
             if (plab > 0) {
-                sh.pp[g.maxmedia * ((g.savedetflag >> 1) & 1) + plab - 1] += f.z;
+                atomicAdd(&sh.pp[g.maxmedia * ((ft & kfCountTally) ? 1u : 0u) + plab - 1], f.z);
             }
         }
 
-        mediaidold = s.mediaid | isdet;
-        idx1dold = s.idx1d;
-        s.idx1d = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+        /* a photon that left its voxel deposits there; one crossing out of a background
+           voxel keeps label 0 (src/mcx_core.cl:2806-2930) */
+        const bool moved = (cross | (FULL && hitintf)) & (oidx < g.nvox) & ((omed | isdet) != 0);
+        const uint32_t flag = isdet;
+        BoxCell* cell = sh.box;
+        float boxold = 0.f;
+        uint32_t gaddr = 0, out_a = 0;
+        double out_v = 0.0;
+        bool evict = false;
 
-        if (!inside(g, s.fx, s.fy, s.fz)) {
-            s.mediaid = 0;
-            s.idx1d = (s.fx < 0 || s.fy < 0 || s.fz < 0) ? K_OUT_MIN : K_OUT_MAX;
-            isdet = g.bc[(s.idx1d == K_OUT_MAX) * 3 + face];
-            isdet = ((isdet & 0xF) == 0) ? (g.doreflect ? (uint32_t)kReflect : (uint32_t)kAbsorb) : isdet;
+        /* the deposit: computed for every lane, most of a wave's lanes deposit in most
+           steps */
+        float weight = 0.f, weight_im = 0.f;
+        int tshift = gate_of(g, f.y);
+        bool deposits = moved & ((ft & kfSave) != 0) & (f.y >= g.twin0) & (f.y < g.twin1);
+
+        if (FULL && (ft & kfRf)) {
+            /* RF forward (src/mcx_core.cl:2833-2839): (w0 - w) / (mua + i omega n / c0) */
+            const float w0re = sh.pp[g.rfoff], w0im = sh.pp[g.rfoff + 1];
+            const float dre = w0re - rf.wre, dim = w0im - rf.wim;
+            const float aim = g.omega * s.prop.w * g.oneoverc0;
+            const float amag2 = s.prop.x * s.prop.x + aim * aim;
+            weight = (amag2 < K_EPS) ? (w0re * pathlen) : kdiv(dre * s.prop.x + dim * aim, amag2);
+            weight_im = (amag2 < K_EPS) ? (w0im * pathlen) : kdiv(dim * s.prop.x - dre * aim, amag2);
+        } else if (ft & kfFlux) {
+            float q = kdiv(s.w0 - p.w, s.prop.x);
+            K_PIN(q);
+            weight = (s.prop.x < K_EPS) ? (s.w0 * pathlen) : q;
+        } else if (g.outputtype == kEnergy) {
+            weight = s.w0 - p.w;
+        } else if (!SIMPLE && g.seed == K_SEED_FROM_FILE) {
+            if (deposits && (g.outputtype == kJacobian || (FULL && (g.outputtype == kRF || g.outputtype == kWLTOF)))) {
+                /* replay path deposits (src/mcx_core.cl:2845-2858): w L (J),
+                   -w L e^{i omega tof} (RF), tof w L (WLTOF) */
+                uint32_t pid = photon_index(g, idx, f.w) - 1;
+                weight = g.replayweight[pid] * pathlen;
+                tshift = gate_of(g, g.replaytof[pid]) +
+                         ((g.replaydet == -1) ? (((g.replaydetid[pid] & 0xFFFF) - 1) * (int)g.maxgate) : 0);
+
+                if (FULL && g.outputtype == kRF) {
+                    weight_im = -weight * sh.pp[g.w0offset + g.srcnum + 1];
+                    weight = -weight * sh.pp[g.w0offset + g.srcnum];
+                } else if (FULL && g.outputtype == kWLTOF) {
+                    weight = weight * g.replaytof[pid];
+                }
+            }
+        } else if (g.outputtype == kL) {
+            weight = s.w0 * pathlen;
+        }
+
+        if (!SIMPLE && (ft & kfSlots)) {
+            tshift += ((int)sh.pp[g.w0offset - 1] - 1) * ((g.replaydet == -1) ? (int)g.detnum : 1) *
+                      (int)g.maxgate;
+        }
+
+        deposits = deposits & (fabsf(weight) > 0.f);
+
+        if (FULL && (ft & kfPatterns)) {
+            if (deposits) {
+            /* several patterns share the photon: one interleaved slot per pattern
+               (src/mcx_core.cl:2902-2914), straight to the grid */
+            const uint32_t base = (oidx + (uint32_t)tshift * g.nvox) * g.npattern;
+
+            for (uint32_t i = 0; i < g.npattern; i++) {
+                const float pw = sh.pp[g.w0offset + i];
+
+                if (fabsf(pw) > 0.f) {
+                    deposit(g, sh.repoff, base + i, weight * pw);
+                }
+            }
+            }
         } else {
-            s.mediaid = g.media[s.idx1d];
-            isdet = s.mediaid & K_DET_MASK;
-            s.mediaid &= K_MED_MASK;
+            const uint32_t dx = (uint32_t)(cx - (int)g.box_x0), dy = (uint32_t)(cy - (int)g.box_y0);
+            const uint32_t dz = (uint32_t)(cz - (int)g.box_z0);
+            const bool inbox = (dx < g.box_nx) & (dy < g.box_ny) & (dz < g.box_nz) & ((uint32_t)tshift < g.box_ng) &
+                               (lin0 == oidx);
+            gaddr = oidx + (uint32_t)tshift * g.nvox;
+
+            if (deposits & inbox) {
+                cell = sh.box + box_offset(g, (uint32_t)tshift, dx, dy, dz);
+#if MCX_PARITY
+                atomicAdd(cell, (BoxCell)weight);
+#else
+                boxold = atomicAdd(cell, weight);
+#endif
+            }
+
+            if (deposits & !inbox) {
+                evict = depcache_add(dcache, gaddr, weight, out_a, out_v);
+            }
+
+            /* a pattern source's deposit carries no imaginary term in the
+               reference (src/mcx_core.cl:2902-2914): its RF forward field
+               stays real */
+            if (FULL && (ft & kfRf) && deposits && g.srctype != kPattern && g.srctype != kPattern3D) {
+                deposit_voxel_im(g, sh, (lin0 == oidx) ? cx : -1, cy, cz, oidx, tshift, weight_im);
+            }
         }
 
-        if ((s.idx1d != idx1dold || (FULL && hitintf)) && idx1dold < g.nvox && mediaidold) {
-            if (g.save2pt && f.y >= g.twin0 && f.y < g.twin1) {
-                float weight = 0.f, weight_im = 0.f;
-                int tshift = gate_of(g, f.y);
+        if (FULL && (ft & kfRfReplay) && moved && f.y >= g.twin0 && f.y < g.twin1 && (ft & kfSave) &&
+                fabsf(weight_im) > 0.f) {
+            deposit(g, sh.repoff, oidx + (uint32_t)tshift * g.nvox + g.imoff, weight_im);
+        }
 
-                if (FULL && g.rfforward) {
-                    /* RF forward (src/mcx_core.cl:2833-2839): (w0 - w) / (mua + i omega n / c0) */
-                    const float w0re = sh.pp[g.rfoff], w0im = sh.pp[g.rfoff + 1];
-                    const float dre = w0re - rf.wre, dim = w0im - rf.wim;
-                    const float aim = g.omega * s.prop.w * g.oneoverc0;
-                    const float amag2 = s.prop.x * s.prop.x + aim * aim;
-                    weight = (amag2 < K_EPS) ? (w0re * pathlen) : kdiv(dre * s.prop.x + dim * aim, amag2);
-                    weight_im = (amag2 < K_EPS) ? (w0im * pathlen) : kdiv(dim * s.prop.x - dre * aim, amag2);
-                } else if (g.outputtype == kEnergy) {
-                    weight = s.w0 - p.w;
-                } else if (g.outputtype == kFluence || g.outputtype == kFlux) {
-                    weight = (s.prop.x < K_EPS) ? (s.w0 * pathlen) : kdiv(s.w0 - p.w, s.prop.x);
-                } else if (!SIMPLE && g.seed == K_SEED_FROM_FILE) {
-                    if (g.outputtype == kJacobian || (FULL && (g.outputtype == kRF || g.outputtype == kWLTOF))) {
-                        /* replay path deposits (src/mcx_core.cl:2845-2858): w L (J),
-                           -w L e^{i omega tof} (RF), tof w L (WLTOF) */
-                        uint32_t pid = photon_index(g, idx, f.w) - 1;
-                        weight = g.replayweight[pid] * pathlen;
-                        tshift = gate_of(g, g.replaytof[pid]) +
-                                 ((g.replaydet == -1) ? (((g.replaydetid[pid] & 0xFFFF) - 1) * (int)g.maxgate) : 0);
+        K_PIN(dcache.a0);
+        K_PIN(dcache.a1);
+        K_PIN(dcache.v0);
+        K_PIN(dcache.v1);
+        s.w0 = moved ? p.w : s.w0;
+        pathlen = moved ? 0.f : pathlen;
 
-                        if (FULL && g.outputtype == kRF) {
-                            weight_im = -weight * sh.pp[g.w0offset + g.srcnum + 1];
-                            weight = -weight * sh.pp[g.w0offset + g.srcnum];
-                        } else if (FULL && g.outputtype == kWLTOF) {
-                            weight = weight * g.replaytof[pid];
-                        }
-                    }
-                } else if (g.outputtype == kL) {
-                    weight = s.w0 * pathlen;
-                }
+        if (FULL && (ft & kfRf) && moved) {
+            sh.pp[g.rfoff] = rf.wre;
+            sh.pp[g.rfoff + 1] = rf.wim;
+        }
 
-                if (!SIMPLE && g.extrasrclen && g.srcid < 0) {
-                    tshift += ((int)sh.pp[g.w0offset - 1] - 1) * ((g.replaydet == -1) ? (int)g.detnum : 1) *
-                              (int)g.maxgate;
-                }
+        bool reflected = false;
 
-                if (FULL && g.npattern > 1) {
-                    /* several patterns share the photon: one interleaved slot per pattern
-                       (src/mcx_core.cl:2902-2914), straight to the grid */
-                    const uint32_t base = (idx1dold + (uint32_t)tshift * g.nvox) * g.npattern;
+        /* the wait for the label belongs here, ahead of the grid atomic: the counter that
+           the wait uses also counts atomics, and this one then has until the next label
+           to complete */
+        K_PIN(lab);
 
-                    for (uint32_t i = 0; i < g.npattern; i++) {
-                        const float pw = sh.pp[g.w0offset + i];
+        if (evict) {
+            grid_add(g, sh.repoff + out_a, out_v);
+        }
 
-                        if (fabsf(pw) > 0.f && fabsf(weight) > 0.f) {
-                            deposit(g, sh.repoff, base + i, weight * pw);
-                        }
-                    }
-                } else if (fabsf(weight) > 0.f) {
-                    deposit_voxel(g, sh, dcache, ox, oy, oz, idx1dold, tshift, weight);
+        s.mediaid = (cross & moved) ? (lab & K_MED_MASK) : s.mediaid;
 
-                    /* a pattern source's deposit carries no imaginary term in the
-                       reference (src/mcx_core.cl:2902-2914): its RF forward field
-                       stays real */
-                    if (FULL && g.rfforward && g.srctype != kPattern && g.srctype != kPattern3D) {
-                        deposit_voxel_im(g, sh, ox, oy, oz, idx1dold, tshift, weight_im);
-                    }
-                }
-
-                if (FULL && g.outputtype == kRF && g.seed == K_SEED_FROM_FILE && g.omega > 0.f &&
-                        fabsf(weight_im) > 0.f) {
-                    deposit(g, sh.repoff, idx1dold + (uint32_t)tshift * g.nvox + g.imoff, weight_im);
-                }
-            }
-
-            s.w0 = p.w;
-
-            if (FULL && g.rfforward) {
-                sh.pp[g.rfoff] = rf.wre;
-                sh.pp[g.rfoff + 1] = rf.wim;
-            }
-
-            pathlen = 0.f;
+        if (SAVEDET) {
+            isdet = cross ? (lab & K_DET_MASK) : ((FULL && hitintf) ? detvox : (isdet | detvox));
         } else {
-            s.mediaid = mediaidold;
+            isdet = 0;
         }
 
-        if (FULL && g.svmc) {
+        if (cross & !in) {
+            isdet = ((s.idx1d == K_OUT_MAX ? bcmax : bcmin) >> (8 * face)) & 0xFFu;
+        }
+
+        if (FULL && (ft & kfSvmc)) {
             /* split voxels (src/mcx_core.cl:2937-2949): a new voxel brings its own
                plane and side; a plane crossing moves the photon to the other side */
-            if (s.idx1d != idx1dold) {
+            if (cross) {
                 s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
                 testint = true;
             } else if (hitintf) {
@@ -1959,11 +2157,45 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 
         /* split voxels also end the photon on entering label 0 through a voxel face
            or the plane, unless it can reflect there (src/mcx_core.cl:2959-2966) */
-        const bool svexit = FULL && g.svmc && (s.idx1d != idx1dold || hitintf) && !K_SV_ISUPPER(s.sv) &&
-                            !K_SV_LOWER(s.sv) && (!g.doreflect || n1 == sh.prop[0].w);
+        const bool svexit = FULL && (ft & kfSvmc) && (cross || hitintf) && !K_SV_ISUPPER(s.sv) &&
+                            !K_SV_LOWER(s.sv) && (!g.doreflect || n1 == n0);
+        const uint32_t code = isdet & 0xFu;
+        /* the index the photon comes from; the properties become the new voxel's (a
+           reflection reads the old ones again) */
+        const float nold = n1;
 
-        if ((s.mediaid == 0 && ((isdet & 0xF) == kAbsorb || (isdet & 0xF) == kCyclic ||
-                                ((isdet & 0xF) == kReflect && n1 == sh.prop[0].w))) || svexit || !(f.y <= g.twin1)) {
+        if (cross && !(FULL && (ft & kfSvmc))) {
+            s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+        }
+
+        n1 = s.prop.w;
+#if !MCX_PARITY
+
+        if (fabsf(boxold) > K_BOX_MOVE) {
+            box_move(g, sh, cell, boxold, gaddr);
+        }
+
+#endif
+        const bool ends = ((s.mediaid == 0) & ((code == kAbsorb) | (code == kCyclic) | ((code == kReflect) & (nold == n0)))) |
+                          svexit | !(f.y <= g.twin1);
+        const bool mirror = code == kMirror;
+        bool rare = ends | (fabsf(p.w) < g.minenergy);
+
+        if (REFLECT) {
+            rare = rare | mirror | (nold != n1) | (FULL && hitintf) | (FULL && (ft & kfMoveOnly));
+        }
+
+        if (!rare) {
+            if (SAVEDET) {
+                detvox = cross ? isdet : detvox;
+            }
+
+            continue;
+        }
+
+        if (ends) {
+            bool wrapped = false;
+
             if (isdet == kCyclic) {
                 if (face == 0) {
                     p.x = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_x : 0.f), (v.x > 0.f) - (v.x < 0.f));
@@ -1982,17 +2214,30 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 
                 if (inside(g, s.fx, s.fy, s.fz)) {
                     s.idx1d = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
-                    s.mediaid = g.media[s.idx1d];
+                    s.mediaid = media_at(g, s.idx1d);
                     isdet = s.mediaid & K_DET_MASK;
+                    detvox = isdet;
                     s.mediaid &= K_MED_MASK;
-                    continue;
+                    lin = s.idx1d;
+                    /* the next step still compares with the index of the voxel left here,
+                       as in the reference */
+                    n1 = nold;
+
+                    if (!(FULL && (ft & kfSvmc))) {
+                        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+                    }
+
+                    wrapped = true;
                 }
             }
 
-            launchflag = (((s.idx1d == K_OUT_MAX && g.bc[9 + face]) || (s.idx1d == K_OUT_MIN && g.bc[6 + face])) ?
-                          K_OUT_MIN : (mediaidold & K_DET_MASK));
-            relaunch = true;
-            testint = testint || (FULL && g.svmc);
+            if (!wrapped) {
+                launchflag = (((s.idx1d == K_OUT_MAX && ((bcdet >> (3 + face)) & 1u)) ||
+                               (s.idx1d == K_OUT_MIN && ((bcdet >> face) & 1u))) ? K_OUT_MIN : flag);
+                relaunch = true;
+                testint = testint || (FULL && (ft & kfSvmc));
+            }
+
             continue;
         }
 
@@ -2007,7 +2252,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     sh.pp[g.rfoff + 1] *= K_ROULETTE;
                 }
             } else {
-                launchflag = mediaidold & K_DET_MASK;
+                launchflag = flag;
                 relaunch = true;
                 continue;
             }
@@ -2016,7 +2261,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         if (REFLECT) {
             bool atface = true;
 
-            if (FULL && g.svmc) {
+            if (FULL && (ft & kfSvmc)) {
                 /* split voxels keep the properties of the side taken above; at the
                    plane, Fresnel reflection or refraction between the two labels
                    (src/mcx_core.cl:3072-3110) replaces the voxel-face test */
@@ -2029,8 +2274,8 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                         s.sn[2] = -s.sn[2];
                         s.sn[3] = -s.sn[3];
 
-                        if (svmc_reflect(n1, v, s, sh.prop, rng)) {
-                            launchflag = mediaidold & K_DET_MASK;
+                        if (svmc_reflect(nold, v, s, sh.prop, rng)) {
+                            launchflag = flag;
                             relaunch = true;
                             testint = true;
                             continue;
@@ -2039,36 +2284,34 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                         s.prop = sh.prop[K_SV_CURLABEL(s.sv)];
                     }
                 }
-            } else {
-                s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d);
             }
 
-            if (atface && ((s.mediaid && g.doreflect) ||
-                    (s.mediaid == 0 && (((isdet & 0xF) == 0 && g.doreflect) || ((isdet & 0xF) == kReflect ||
-                                        (isdet & 0xF) == kMirror)))) &&
-                    (((isdet & 0xF) == kMirror) || n1 != s.prop.w)) {
+            const bool doref = (ft & kfReflect) != 0;
+
+            if (atface && (mirror | (nold != s.prop.w)) &&
+                    (s.mediaid ? doref : ((code == 0) & doref) | (code == kReflect) | mirror)) {
                 float Rtotal = 1.f;
                 float cphi, sphi, stheta, ctheta;
-                float tmp0 = n1 * n1;
+                float tmp0 = nold * nold;
                 float tmp1 = s.prop.w * s.prop.w;
                 cphi = fabsf((face == 0) ? v.x : (face == 1 ? v.y : v.z));
                 sphi = 1.f - cphi * cphi;
                 f.z = 1.f - kdiv(tmp0, tmp1) * sphi;
 
-                if (f.z > 0.f && (isdet & 0xF) != kMirror) {
+                if (f.z > 0.f && !mirror) {
                     ctheta = tmp0 * cphi * cphi + tmp1 * f.z;
-                    stheta = 2.f * n1 * s.prop.w * cphi * ksqrt(f.z);
+                    stheta = 2.f * nold * s.prop.w * cphi * ksqrt(f.z);
                     Rtotal = kdiv(ctheta - stheta, ctheta + stheta);
                     ctheta = tmp1 * cphi * cphi + tmp0 * f.z;
                     Rtotal = (Rtotal + kdiv(ctheta - stheta, ctheta + stheta)) * 0.5f;
                 }
 
-                if (Rtotal < 1.f && (!(s.mediaid == 0 && ((isdet & 0xF) == kMirror))) && rng.next() > Rtotal) {
-                    transmit(v, n1, s.prop.w, face);
+                if (Rtotal < 1.f && (!(s.mediaid == 0 && mirror)) && rng.next() > Rtotal) {
+                    transmit(v, nold, s.prop.w, face);
 
                     if (s.mediaid == 0) {
-                        launchflag = (((s.idx1d == K_OUT_MAX && g.bc[9 + face]) ||
-                                       (s.idx1d == K_OUT_MIN && g.bc[6 + face])) ? K_OUT_MIN : (mediaidold & K_DET_MASK));
+                        launchflag = (((s.idx1d == K_OUT_MAX && ((bcdet >> (3 + face)) & 1u)) ||
+                                       (s.idx1d == K_OUT_MIN && ((bcdet >> face) & 1u))) ? K_OUT_MIN : flag);
                         relaunch = true;
                         continue;
                     }
@@ -2087,63 +2330,73 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                         s.fz = to_short((int)rintf(p.z));
                     }
 
-                    s.idx1d = idx1dold;
-                    keepold = true;
-                    /* back in the voxel it came from, whose label mediaidold holds
-                       (the reference reloads it from the volume) */
-                    s.mediaid = mediaidold & K_MED_MASK;
+                    /* back in the voxel it came from, with its label and properties */
+                    s.idx1d = oidx;
+                    s.mediaid = omed;
+                    reflected = true;
+                    lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
 
-                    if (FULL && g.svmc) {
+                    if (!(FULL && (ft & kfSvmc))) {
+                        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+                    } else {
                         /* the side of the plane the reflected photon lands on; label 0
                            there ends it (src/mcx_core.cl:3221-3243) */
                         s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
 
                         if (K_SV_CURLABEL(s.sv) == 0) {
-                            launchflag = mediaidold & K_DET_MASK;
+                            launchflag = flag;
                             relaunch = true;
                             continue;
                         }
-                    } else {
-                        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d);
                     }
 
-                    n1 = s.prop.w;
                     /* drop the boundary code so a later same-voxel step restores
                        the voxel's own label (the reference ORs the code in) */
                     isdet &= K_DET_MASK;
                 }
             }
 
-            if (FULL && g.moveonly && (s.mediaid == 0 || s.idx1d == K_OUT_MIN || s.idx1d == K_OUT_MAX)) {
+            if (FULL && (ft & kfMoveOnly) && (s.mediaid == 0 || s.idx1d == K_OUT_MIN || s.idx1d == K_OUT_MAX)) {
                 /* move-only trajectories (debug flag T, src/mcx_core.cl:3287-3291): the
                    lane's whole run ends here, without its energy write-back */
                 moveend = true;
                 break;
             }
         }
+
+        n1 = s.prop.w;
+
+        if (SAVEDET) {
+            detvox = (cross & !reflected) ? (isdet & K_DET_MASK) : detvox;
+        }
     }
 
     depcache_flush(g, sh, dcache);
+    esc = s.esc;
+    tot = s.tot;
     return !moveend;
 }
 
-#ifdef MCX_WAVES_PER_EU
-#define MCX_KATTR __attribute__((amdgpu_waves_per_eu(MCX_WAVES_PER_EU)))
-#else
-#define MCX_KATTR
-#endif
+/* The fast build runs one workgroup of bound/64 waves per CU, so the instances that
+   need fewer registers than that leaves them are not packed tighter: the deposit
+   box is worth more than a fifth wave per SIMD. */
 #if MCX_PARITY
 #define MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL) MCX_MAX_BLOCK
+#define MCX_KATTR(bound)
 #else
 #define MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL) MCX_FAST_BOUND_FULL(SAVEDET, REFLECT, SIMPLE, FULL)
+#define MCX_KATTR(bound) __attribute__((amdgpu_waves_per_eu((bound) / 256, MCX_FAST_WAVES)))
 #endif
 template <bool SAVEDET, bool REFLECT, bool SIMPLE, bool FULL>
-__global__ void __launch_bounds__(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) MCX_KATTR transport_kernel(const MCXKParam g) {
+__global__ void __launch_bounds__(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL))
+MCX_KATTR(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) transport_kernel(const MCXKParam g) {
     extern __shared__ float4 lds[];
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t pplen = g.pplen;
     __shared__ uint32_t pool[2];
     Shared sh;
+    /* the parameter block is the kernel's only argument: the kernarg segment starts with it */
+    sh.kp = (KParamPtr)__builtin_amdgcn_kernarg_segment_ptr();
     sh.pool = pool;
     sh.prop = lds;
     sh.invcdf = (float*)(lds + g.medianum);
@@ -2187,18 +2440,16 @@ __global__ void __launch_bounds__(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) MC
     const bool active = g.dynamic ? (uint32_t)idx < g.nthread :
                         !((uint32_t)idx >= g.threadphoton * g.nthread + (uint32_t)g.oddphoton ||
                           (uint32_t)idx >= g.nthread);
-    const uint32_t pd = g.partialdata;
     /* the tail workgroup may hold lanes past nthread: they read nothing */
     const uint32_t sidx = (uint32_t)idx < g.nthread ? (uint32_t)idx : 0u;
-    sh.pp[pd] = g.genergy[sidx * 2];
-    sh.pp[pd + 1] = g.genergy[sidx * 2 + 1];
+    float esc = g.genergy[sidx * 2], tot = g.genergy[sidx * 2 + 1];
     Rng rng;
     rng.s0 = (uint64_t)g.nseed[sidx * 4] << 32 | g.nseed[sidx * 4 + 1];
     rng.s1 = (uint64_t)g.nseed[sidx * 4 + 2] << 32 | g.nseed[sidx * 4 + 3];
 
-    if (active && transport_lane<SAVEDET, REFLECT, SIMPLE, FULL>(g, sh, rng, idx)) {
-        g.genergy[idx * 2] = sh.pp[pd];
-        g.genergy[idx * 2 + 1] = sh.pp[pd + 1];
+    if (active && transport_lane<SAVEDET, REFLECT, SIMPLE, FULL>(g, sh, rng, idx, esc, tot)) {
+        g.genergy[idx * 2] = esc;
+        g.genergy[idx * 2 + 1] = tot;
     }
 
     if (g.box_cells) {
@@ -2216,7 +2467,7 @@ __global__ void __launch_bounds__(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) MC
                 uint32_t z = r % g.box_nz, gate = r / g.box_nz;
                 uint32_t vox = (g.box_z0 + z) * g.dimxy + (g.box_y0 + y) * g.dimx + (g.box_x0 + x);
                 gate = (gate < g.box_ng) ? gate : gate - g.box_ng + g.box_imgate;
-                atomicAdd(g.field + boff + vox + gate * g.nvox, val);
+                grid_add(g, boff + vox + gate * g.nvox, val);
             }
         }
     }
@@ -2306,6 +2557,7 @@ __global__ void __launch_bounds__(MCX_BATCH_BLOCK_MAX) __attribute__((amdgpu_wav
         const long long tstart = cost ? wall_clock64() : 0;
         const uint32_t pplen = g.pplen;
         Shared sh;
+        sh.kp = (KParamPtr)(prm + inst);
         sh.pool = pools + 2 * inst;
         sh.prop = lds;
         sh.invcdf = (float*)(lds + g.medianum);
@@ -2333,11 +2585,10 @@ __global__ void __launch_bounds__(MCX_BATCH_BLOCK_MAX) __attribute__((amdgpu_wav
 
         /* the general path only: with the pencil-beam special path inlined beside
            it the kernel needs more registers and runs fewer waves per SIMD */
-        transport_lane<false, REFLECT, false, false>(g, sh, rng, lane);
+        float lesc = 0.f, ltot = 0.f;
+        transport_lane<false, REFLECT, false, false>(g, sh, rng, lane, lesc, ltot);
 
-        const uint32_t pd = g.partialdata;
-        double esc = wave_sum((double)sh.pp[pd]);
-        double tot = wave_sum((double)sh.pp[pd + 1]);
+        const double esc = wave_sum((double)lesc), tot = wave_sum((double)ltot);
 
         if ((threadIdx.x & 63) == 0 && tot != 0.0) {
             atomicAdd(energy + 2 * inst, esc);
@@ -2355,7 +2606,7 @@ __global__ void __launch_bounds__(MCX_BATCH_BLOCK_MAX) __attribute__((amdgpu_wav
                 r /= g.box_ny;
                 uint32_t z = r % g.box_nz, gate = r / g.box_nz;
                 uint32_t vox = (g.box_z0 + z) * g.dimxy + (g.box_y0 + y) * g.dimx + (g.box_x0 + x);
-                atomicAdd(g.field + vox + gate * g.nvox, val);
+                grid_add(g, vox + gate * g.nvox, val);
             }
         }
 

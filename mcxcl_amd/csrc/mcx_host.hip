@@ -300,8 +300,11 @@ void mcx_check_supported(const Config* cfg) {
 /* kernel parameters of one simulation on nthread lanes in workgroups of lblock:
    geometry, time gates, record layout, the specialised-path flag, the LDS deposit
    box and the accumulator replicas.  Returns the dynamic LDS bytes per workgroup;
-   *reflect receives the reference's rule for the reflection kernel variant. */
-size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lblock, int* reflect, size_t boxbytes) {
+   *reflect receives the reference's rule for the reflection kernel variant;
+   pencil allows the pencil path's shorter lane scratch (the batched kernel always
+   runs the general path). */
+size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lblock, int* reflect, size_t boxbytes,
+                        int pencil) {
     const unsigned int maxgate = (unsigned int)((cfg->tend - cfg->tstart) / cfg->tstep + 0.5);
     cfg->maxgate = maxgate;
     const size_t nvox = (size_t)cfg->dim.x * cfg->dim.y * cfg->dim.z;
@@ -367,7 +370,7 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
     g.savedetflag = cfg->savedetflag;
     g.reclen = reclen;
     g.partialdata = partialdata;
-    g.w0offset = partialdata + 4;
+    g.w0offset = partialdata + 2;
     g.gscatter = cfg->gscatter;
     g.srcnum = cfg->srcnum;
     g.doreflect = (uint32_t)cfg->isreflect;
@@ -386,7 +389,7 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
     g.nangle = cfg->nangle;
     g.imoff = isrf ? (uint32_t)halflen : 0u;
     g.omega = cfg->omega;
-    /* lane scratch: record columns, 2 tallies, w0, source id, one weight per
+    /* lane scratch: record columns, w0, source id, one weight per
        shared pattern (srcnum), the RF replay phase (cos, sin) */
     g.pplen = g.w0offset + g.srcnum + (isrfreplay ? 2u : 0u);
     /* polarised runs: the Stokes vector after them */
@@ -465,11 +468,21 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
         }
     }
 
-    size_t pplen = g.pplen;
-    size_t shmem = cfg->medianum * sizeof(float4) + ((cfg->nphase + 3) & ~3u) * sizeof(float) +
-                   lblock * pplen * sizeof(float);
+    const size_t tables = cfg->medianum * sizeof(float4) + ((cfg->nphase + 3) & ~3u) * sizeof(float);
+    /* the stated limit counts two energy tallies per lane, which live in registers now */
+    const size_t limit = tables + (pencil && lblock > MCX_LAUNCH_BLOCK ? MCX_LAUNCH_BLOCK : lblock) *
+                         ((size_t)g.pplen + 2) * sizeof(float);
 
-    if (shmem + MCX_LDS_SLACK > MCX_LDS_LIMIT) {
+    if (pencil && g.simple) {
+        /* the pencil beam's launch weight is the source's, its source the only one */
+        g.seedoff = partialdata;
+        g.pplen = partialdata + ((cfg->issaveseed > 0) ? 4u : 0u);
+    }
+
+    const size_t pplen = g.pplen;
+    size_t shmem = tables + lblock * pplen * sizeof(float);
+
+    if ((limit > shmem ? limit : shmem) + MCX_LDS_SLACK > MCX_LDS_LIMIT) {
         MCX_ERROR(-4, "too many media/phase samples or record columns for the LDS tables");
     }
 
@@ -662,7 +675,7 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
     MCXKParam& g = *gp;
     int reflect = 0;
     size_t nthread = *nthread_io;
-    size_t shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, fast ? 0 : MCX_BOX_BYTES);
+    size_t shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, fast ? 0 : MCX_BOX_BYTES, 1);
     {
         const size_t bound = fast ? (size_t)MCX_FAST_BOUND_FULL(cfg->issavedet != 0, reflect != 0, g.simple != 0,
                                  g.full != 0) : MCX_MAX_BLOCK;
@@ -692,7 +705,7 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
             MCX_ERROR(-99, "cannot select the HIP device");
         }
 
-        shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, 0);
+        shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, 0, 1);
 
         if (hipDeviceGetAttribute(&ldscu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) == hipSuccess &&
                 hipDeviceGetAttribute(&ldsblock, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess) {
@@ -701,7 +714,7 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
             if (nwg <= 0 && dynamic && !envblock && lblock > MCX_MAX_BLOCK) {
                 /* no CU holds the wide workgroup: fall back to 256 lanes */
                 lblock = MCX_MAX_BLOCK;
-                shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, 0);
+                shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, 0, 1);
                 nwg = mcx_fast_occupancy((int)lblock, shmem, cfg->issavedet != 0, reflect, g.full ? 2 : (int)g.simple);
             }
         }
@@ -715,7 +728,7 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
             budget = per > shmem + MCX_LDS_SLACK ? per - shmem - MCX_LDS_SLACK : 0;
         }
 
-        shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, budget);
+        shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, budget, 1);
     }
 
     size_t nlaunch = (nthread + lblock - 1) / lblock;
