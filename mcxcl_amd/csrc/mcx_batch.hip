@@ -85,6 +85,8 @@ struct MCXBatch {
     uint32_t* dqlist;
     uint32_t* dstate;
     uint32_t* dstate0;
+    uint32_t* dhand;                /* hand-over slots of the workgroups' thinned-out waves */
+    uint32_t handwords;             /* words a lane moves there, the largest instance's */
     unsigned long long* dcost;      /* per-instance workgroup time of a probe step */
     uint32_t nqueue, nstate;
     size_t lblock, nblock, shmem;
@@ -292,7 +294,7 @@ static void batch_enqueue(MCXBatch* b, int timed, int probe) {
     }
 
     BHIP(mcx_launch_batch(b->dprm, b->dqlist, b->nqueue, b->dstate, b->dnseed, b->denergy, probe ? b->dcost : NULL,
-                          (int)b->nblock, (int)b->lblock, b->shmem, b->reflect, b->stream));
+                          b->dhand, b->handwords, (int)b->nblock, (int)b->lblock, b->shmem, b->reflect, b->stream));
 
     if (timed) {
         BHIP(hipEventRecord(b->ev2, b->stream));
@@ -440,6 +442,7 @@ static void batch_create_impl(MCXBatch* b, Config** cfgs, unsigned int n, MCXBat
         MCXKParam g;
         int reflect;
         (void)mcx_kparam_setup(cfg, &g, 64, 64, &reflect, 0, 0);
+        b->handwords = b->handwords > MCX_HAND_WORDS + g.pplen ? b->handwords : MCX_HAND_WORDS + g.pplen;
         b->fieldoff[i + 1] = b->fieldoff[i] + g.fieldlen;
         maxlen = g.fieldlen > maxlen ? g.fieldlen : maxlen;
         nvoxall += g.nvox;
@@ -503,6 +506,7 @@ static void batch_create_impl(MCXBatch* b, Config** cfgs, unsigned int n, MCXBat
     b->dstate0 = batch_alloc<uint32_t>(b, b->nstate);
     b->denergy = batch_alloc<double>(b, 2 * (size_t)n);
     b->dcost = batch_alloc<unsigned long long>(b, n);
+    b->dhand = batch_alloc<uint32_t>(b, b->maxlanes / 4 * b->handwords);
     b->dnseed = batch_alloc<uint32_t>(b, b->maxlanes * 4);
     BHIP(hipMemcpyAsync(b->dnorm, b->norm, n * sizeof(MCXBatchNorm), hipMemcpyHostToDevice, b->stream));
 

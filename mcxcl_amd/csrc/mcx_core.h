@@ -13,11 +13,15 @@
    launches 256-lane workgroups.  The fast build runs one workgroup per CU, so
    that a single LDS deposit box can use most of the CU's LDS instead of being
    split between several workgroups: 1024 lanes (16 waves, <=128 VGPRs) for the
-   pencil-beam specialisation (109 VGPRs) and for the general path without
-   detected photons or without reflection (7-9 VGPRs spilled to scratch, still
-   6-9% faster than 768 lanes), 768 lanes (12 waves, <=168 VGPRs, no spills)
-   for the general path with both, which would spill 21. */
+   pencil-beam specialisation (101 VGPRs) and for the general path without
+   detected photons or without reflection (11-13 VGPRs spilled to scratch outside
+   the step loop, 6-9% faster than 768 lanes), 768 lanes (12 waves, <=168 VGPRs, no
+   spills) for the general path with both (152 VGPRs). */
 #define MCX_MAX_BLOCK 256
+/* a wave hands its lanes over once at most this many are live (a quarter: the lanes of
+   four waves fit in one), and the words a lane moves besides its LDS scratch */
+#define MCX_HAND_LANES 16u
+#define MCX_HAND_WORDS 42u
 #define MCX_FAST_SIMPLE_BLOCK 1024
 /* waves per SIMD the fast kernels are built for (amdgpu_waves_per_eu caps them) */
 #define MCX_FAST_WAVES 4
@@ -73,6 +77,7 @@ struct MCXKParam {
                                      (0: real output) */
     float omega;                  /* angular modulation frequency, rad/s */
     uint32_t rfforward;           /* 1: complex photon weights and fluence (omega > 0 without replay) */
+    uint32_t blocklanes;          /* lanes of the thread map per workgroup (at most its threads) */
     uint32_t dynamic;             /* 1: photons are handed out per workgroup at run time
                                      (threadphoton/oddphoton then split photons over workgroups) */
     uint32_t simple;              /* 1: pencil beam from a non-void voxel without focus, extra sources,
@@ -115,6 +120,7 @@ struct MCXKParam {
     uint64_t* detseed;            /* 2 words per detected photon */
     uint32_t* detcount;
     float* debugdata;             /* trajectory records: {photon id bits, x, y, z, w, source id} */
+    uint32_t* hand;               /* hand-over slots of the workgroups' thinned-out waves; NULL: none */
     uint32_t* jumpdebug;          /* trajectory records written, counted past maxjumpdebug */
 };
 
@@ -149,8 +155,8 @@ hipError_t mcx_launch_atomic_probe(double* grid, uint32_t n, uint32_t nblock, ui
 hipError_t mcx_launch_rngdump(const MCXKParam* prm, int nblock, int nthreadblock, hipStream_t stream);
 /* batched launch: many simulations in one persistent kernel (fast arithmetic) */
 hipError_t mcx_launch_batch(const MCXKParam* prm, const uint32_t* qlist, uint32_t nqueue, uint32_t* state,
-                            uint32_t* nseed, double* energy, unsigned long long* cost, int nblock, int nthreadblock,
-                            size_t shmem, int reflect, hipStream_t stream);
+                            uint32_t* nseed, double* energy, unsigned long long* cost, uint32_t* hand, uint32_t handwords, int nblock,
+                            int nthreadblock, size_t shmem, int reflect, hipStream_t stream);
 int mcx_batch_occupancy(int nthreadblock, size_t shmem, int reflect);
 hipError_t mcx_launch_batch_prep(double* field, size_t nfield, double* energy, uint32_t nenergy, uint32_t* state,
                                  const uint32_t* state0, uint32_t nstate, hipStream_t stream);

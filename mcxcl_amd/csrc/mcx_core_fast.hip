@@ -84,14 +84,14 @@ extern "C" int mcx_fast_occupancy(int nthreadblock, size_t shmem, int savedet, i
 
 /* ---------------- batched launch ---------------- */
 extern "C" hipError_t mcx_launch_batch(const MCXKParam* prm, const uint32_t* qlist, uint32_t nqueue, uint32_t* state,
-                                       uint32_t* nseed, double* energy, unsigned long long* cost, int nblock,
-                                       int nthreadblock, size_t shmem, int reflect, hipStream_t stream) {
+                                       uint32_t* nseed, double* energy, unsigned long long* cost, uint32_t* hand,
+                                       uint32_t handwords, int nblock, int nthreadblock, size_t shmem, int reflect, hipStream_t stream) {
     if (reflect) {
         hipLaunchKernelGGL(mcxk::batch_kernel<true>, dim3(nblock), dim3(nthreadblock), shmem, stream, prm, qlist,
-                           nqueue, state, nseed, energy, cost);
+                           nqueue, state, nseed, energy, cost, hand, handwords);
     } else {
         hipLaunchKernelGGL(mcxk::batch_kernel<false>, dim3(nblock), dim3(nthreadblock), shmem, stream, prm, qlist,
-                           nqueue, state, nseed, energy, cost);
+                           nqueue, state, nseed, energy, cost, hand, handwords);
     }
 
     return hipGetLastError();

@@ -79,6 +79,9 @@ __device__ __forceinline__ float klog(float x) {
 __device__ __forceinline__ void ksincos(float x, float* s, float* c) {
     pm_sincos(x, s, c);
 }
+__device__ __forceinline__ void ksincos_turn(float r, float* s, float* c) {
+    pm_sincos(K_TWO_PI * r, s, c);
+}
 __device__ __forceinline__ float ksin(float x) {
     return pm_sin(x);
 }
@@ -106,6 +109,11 @@ __device__ __forceinline__ float klog(float x) {
 }
 __device__ __forceinline__ void ksincos(float x, float* s, float* c) {
     float r = x * 0.159154943091895336f;   /* v_sin/v_cos take revolutions */
+    *s = __builtin_amdgcn_sinf(r);
+    *c = __builtin_amdgcn_cosf(r);
+}
+/* sine and cosine of r turns: the hardware takes turns */
+__device__ __forceinline__ void ksincos_turn(float r, float* s, float* c) {
     *s = __builtin_amdgcn_sinf(r);
     *c = __builtin_amdgcn_cosf(r);
 }
@@ -347,7 +355,11 @@ struct Shared {
     float* invcdf;
     BoxCell* box;                /* privatised deposit box (box_cells) */
     float* pp;                   /* this lane's scratch: partial data, energies, w0, srcid */
-    size_t repoff;               /* offset of this lane's global accumulator replica */
+    size_t repoff;               /* offset of this workgroup's global accumulator replica */
+    uint32_t* wlive;             /* live lanes per wave, for the hand-over (LDS) */
+    uint32_t* hand;              /* this workgroup's hand-over slots (global memory): word k of slot j at
+                                    [k * handslots + j]; NULL: no hand-over */
+    double* energy;              /* batched launch: the workgroup's {escaped, launched} weight (LDS) */
     uint32_t* pool;              /* dynamic schedule: {next photon, end} of this workgroup (LDS)
                                     or of this instance (global memory, batched launch) */
 };
@@ -626,7 +638,7 @@ __device__ __forceinline__ int svmc_reflect(float n1, float4& v, Photon& s, cons
 enum {kfGscatter = 1u << 0, kfPerVoxel = 1u << 1, kfPacked = 1u << 2, kfSvmc = 1u << 3, kfRf = 1u << 4,
       kfSave = 1u << 5, kfFlux = 1u << 6, kfReflect = 1u << 7, kfPathTally = 1u << 8, kfPatterns = 1u << 9,
       kfSlots = 1u << 10, kfMoveOnly = 1u << 11, kfPhase = 1u << 12, kf2D = 1u << 13, kfPol = 1u << 14,
-      kfScatDeposit = 1u << 15, kfTraj = 1u << 16, kfCountTally = 1u << 17, kfMomTally = 1u << 18, kfRfReplay = 1u << 19
+      kfScatDeposit = 1u << 15, kfTraj = 1u << 16, kfCountTally = 1u << 17, kfMomTally = 1u << 18, kfRfReplay = 1u << 19, kfGates = 1u << 20
      };
 
 __device__ __forceinline__ uint32_t features(const MCXKParam& g) {
@@ -653,20 +665,22 @@ __device__ __forceinline__ uint32_t features(const MCXKParam& g) {
     w |= (g.outputtype == kWP || g.outputtype == kDCS || g.outputtype == kWPTOF || (replay && g.outputtype == kRFmus)) ?
          kfScatDeposit : 0u;
     w |= g.savetraj ? kfTraj : 0u;
+    w |= g.maxgate > 1 ? kfGates : 0u;
     w |= (replay && g.outputtype == kRF && g.omega > 0.f) ? kfRfReplay : 0u;
     return w;
 }
 
 /* the properties of the photon's voxel: label table, per-voxel mua/mus
    replacing the label's, or (full general path) a packed media word */
-template <bool FULL = false>
+/* CLEAN: mediaid carries no detector flag */
+template <bool FULL, bool CLEAN>
 __device__ __forceinline__ float4 getprop(const MCXKParam& g, const Shared& sh, uint32_t mediaid, uint32_t idx1d,
         uint32_t ft) {
     if (FULL && (ft & kfPacked)) {
         return media_word_prop(g.mediaformat, sh.prop, mediaid);
     }
 
-    float4 p = sh.prop[mediaid & K_MED_MASK];
+    float4 p = sh.prop[CLEAN ? mediaid : mediaid & K_MED_MASK];
 
     /* per-voxel absorption and scattering: g and n stay those of the label.  The
        label's own values are read first, whatever follows: a select between the LDS
@@ -679,6 +693,10 @@ __device__ __forceinline__ float4 getprop(const MCXKParam& g, const Shared& sh, 
             const K_GLOBAL float* m = (const K_GLOBAL float*)g.muamus + 2 * (size_t)idx1d;
             p.x = m[0];
             p.y = m[1];
+            /* wait here: pending loads at a join make every run wait there, and the counter
+               also holds the grid atomics */
+            K_PIN(p.x);
+            K_PIN(p.y);
         }
     }
 
@@ -1139,7 +1157,7 @@ __device__ __forceinline__ int launch_photon(const MCXKParam& gk, const Shared& 
         s.fy = to_short((int)floorf(p.y));
         s.fz = to_short((int)floorf(p.z));
         f.w += 1.f;
-        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+        s.prop = getprop<FULL, false>(g, sh, s.mediaid, s.idx1d, ft);
         s.tot += p.w;
         s.w0 = p.w;
         v.w = K_EPS;
@@ -1555,7 +1573,7 @@ __device__ __forceinline__ int launch_photon(const MCXKParam& gk, const Shared& 
 
     f.w += 1.f;
     s.prop = (FULL && g.svmc) ? svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s) :
-             getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+             getprop<FULL, false>(g, sh, s.mediaid, s.idx1d, ft);
 
     if (FULL && g.savetraj) {
         save_traj(g, p, traj_index(g, idx, f.w), ppl[1], pp + g.stokesoff);   /* the source-id slot */
@@ -1606,27 +1624,246 @@ __device__ __forceinline__ uint32_t bc_detects(const MCXKParam& g) {
     return w;
 }
 
+/* Hand-over of a thinned-out workgroup.  When the photons to launch have run out, the
+   lanes of a wave end one after the other, and the wave goes on issuing the whole
+   step loop for the few that are left, up to the longest path the time window
+   allows.  So each wave stops once at most MCX_HAND_LANES of its lanes are live
+   (thresh in transport_lane) and meets the workgroup's other waves: the live lanes of
+   all waves move into the first quarter of them, one wave per SIMD of the CU for the
+   fast build's 16, and run to their end there.  A lane moves whole: photon, stream,
+   tallies, LDS scratch and its index in the thread map, so nothing it computes or
+   records depends on where it runs; the lane it leaves takes the other's stream, so
+   every lane goes on with one of its own.  The write-combining entries stay.
+   At most 16 lanes per wave are live, so a quarter of the waves holds them all; the
+   state goes through memory inside the loop (hand_put), which leaves the loop without
+   a copy of it in registers.  Every thread of the workgroup comes here exactly once. */
+struct Moving {
+    float wre, wim, pathlen, n1;
+    uint32_t isdet, detvox, launchflag, lin;
+    bool relaunch, testint;
+};
+
+__device__ __forceinline__ void pin_photon(Photon& s, Rng& rng) {
+    K_PIN(s.p.x);
+    K_PIN(s.p.y);
+    K_PIN(s.p.z);
+    K_PIN(s.p.w);
+    K_PIN(s.v.x);
+    K_PIN(s.v.y);
+    K_PIN(s.v.z);
+    K_PIN(s.v.w);
+    K_PIN(s.f.x);
+    K_PIN(s.f.y);
+    K_PIN(s.f.w);
+    K_PIN(s.prop.x);
+    K_PIN(s.prop.y);
+    K_PIN(s.prop.z);
+    K_PIN(s.prop.w);
+    K_PIN(s.fx);
+    K_PIN(s.fy);
+    K_PIN(s.fz);
+    K_PIN(s.idx1d);
+    K_PIN(s.mediaid);
+    K_PIN(s.sv);
+    K_PIN(s.w0);
+    K_PIN(s.esc);
+    K_PIN(s.tot);
+    K_PIN(rng.s0);
+    K_PIN(rng.s1);
+}
+
+/* the slot of the r-th live lane of wave w, at most MCX_HAND_LANES of them per wave */
+__device__ __forceinline__ uint32_t hand_slot(uint32_t w, uint32_t r) {
+    return w * MCX_HAND_LANES + r;
+}
+
+template <bool PUT>
+__device__ __forceinline__ void hand_copy(const Shared& sh, uint32_t j, Photon& s, Rng& rng, int& idx, Moving& m) {
+    /* hidden from the compiler, which otherwise keeps every word's offset in a scalar
+       register throughout the step loop */
+    uint32_t slots = blockDim.x >> 2, pplen = cold(sh.kp).pplen, k = 0;
+    K_PIN(slots);
+    uint32_t* const slot = sh.hand + j;
+    auto mvu = [&](uint32_t& v) {
+        if (PUT) {
+            slot[k * slots] = v;
+        } else {
+            v = slot[k * slots];
+        }
+
+        k++;
+    };
+    auto mv = [&](float& v) {
+        uint32_t u = __float_as_uint(v);
+        mvu(u);
+        v = __uint_as_float(u);
+    };
+    auto mvi = [&](int& v) {
+        uint32_t u = (uint32_t)v;
+        mvu(u);
+        v = (int)u;
+    };
+    mv(s.p.x), mv(s.p.y), mv(s.p.z), mv(s.p.w);
+    mv(s.v.x), mv(s.v.y), mv(s.v.z), mv(s.v.w);
+    mv(s.f.x), mv(s.f.y), mv(s.f.w);
+    mv(s.prop.x), mv(s.prop.y), mv(s.prop.z), mv(s.prop.w);
+    mvi(s.fx), mvi(s.fy), mvi(s.fz);
+    mvu(s.idx1d), mvu(s.mediaid), mvu(s.sv), mvu(m.isdet), mvu(m.detvox), mvu(m.launchflag), mvu(m.lin);
+    mv(s.w0), mv(s.esc), mv(s.tot), mv(m.pathlen), mv(m.n1), mv(m.wre), mv(m.wim);
+    mvi(idx);
+    uint32_t w[5] = {(m.relaunch ? 1u : 0u) | (m.testint ? 2u : 0u), (uint32_t)rng.s0, (uint32_t)(rng.s0 >> 32),
+                     (uint32_t)rng.s1, (uint32_t)(rng.s1 >> 32)};
+    mvu(w[0]), mvu(w[1]), mvu(w[2]), mvu(w[3]), mvu(w[4]);
+    m.relaunch = w[0] & 1u;
+    m.testint = w[0] & 2u;
+    rng.s0 = (uint64_t)w[2] << 32 | w[1];
+    rng.s1 = (uint64_t)w[4] << 32 | w[3];
+    k += 4;   /* the stream going the other way */
+
+    for (uint32_t i = 0; i < pplen; i++) {
+        mv(sh.pp[i]);
+    }
+}
+
+/* where the stream of the lane that takes slot j waits for the one that left it */
+__device__ __forceinline__ void hand_stream(const Shared& sh, uint32_t j, Rng& rng, bool put) {
+    const uint32_t slots = blockDim.x >> 2;
+    uint32_t* const w = sh.hand + j + (MCX_HAND_WORDS - 4u) * slots;
+
+    if (put) {
+        w[0] = (uint32_t)rng.s0;
+        w[slots] = (uint32_t)(rng.s0 >> 32);
+        w[2 * slots] = (uint32_t)rng.s1;
+        w[3 * slots] = (uint32_t)(rng.s1 >> 32);
+    } else {
+        rng.s0 = (uint64_t)w[slots] << 32 | w[0];
+        rng.s1 = (uint64_t)w[3 * slots] << 32 | w[2 * slots];
+    }
+}
+
+/* put: this lane is live and its state is in its wave's slots.  Returns whether the lane
+   runs on, and in j the slot to take its state from; streams are exchanged here. */
+__device__ __forceinline__ bool hand_over(const Shared& sh, bool put, Rng& rng, uint32_t& j) {
+    uint32_t size = blockDim.x;
+    asm("" : "+s"(size));
+    const uint32_t lane = threadIdx.x & 63u, nwave = size >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t live = __ballot(put), below = (1ull << lane) - 1ull;
+    const uint32_t mine = (uint32_t)__popcll(live);
+
+    if (lane == 0) {
+        sh.wlive[wave] = mine;
+    }
+
+    __syncthreads();
+    /* the first ntake waves take the lanes of the others, up to `even` lanes each */
+    const uint32_t ntake = (nwave + 3) >> 2;
+    uint32_t total = 0, low = 0;
+
+    for (uint32_t w = 0; w < nwave; w++) {
+        const uint32_t n = sh.wlive[w];
+        total += n;
+        low += w < ntake ? n : 0u;
+    }
+
+    const uint32_t even = (total + ntake - 1) / ntake;
+    uint32_t rank = (uint32_t)__popcll((put ? live : ~live) & below);
+    j = hand_slot(wave, rank);
+    bool takes = false;
+
+    if (wave < ntake && !put && rank < (even > mine ? even - mine : 0u)) {
+        /* the rank-th of this wave's share: the lanes before it go to the waves before it */
+        for (uint32_t w = 0; w < wave; w++) {
+            const uint32_t n = sh.wlive[w];
+            rank += even > n ? even - n : 0u;
+        }
+
+        takes = rank < total - low;
+
+        if (takes) {
+            uint32_t w = ntake;
+
+            while (w < nwave - 1 && rank >= sh.wlive[w]) {
+                rank -= sh.wlive[w];
+                w++;
+            }
+
+            j = hand_slot(w, rank);
+            hand_stream(sh, j, rng, true);
+        }
+    }
+
+    __syncthreads();
+
+    if (put && wave >= ntake) {
+        hand_stream(sh, j, rng, false);
+        return false;
+    }
+
+    return put || takes;
+}
+
 /* What bounds the step loop: instruction issue of a wave (most steps of a wave take
-   every branch), then the waits for the label and the grid atomic behind it.  So the
-   state is updated in place under selects (K_PIN), a run's options sit in one scalar
-   register (features), boundary codes in another, rare branches share one test, the
-   label and the properties are read only where the voxel changes, and the energy
-   tallies are registers, which leaves their LDS to the deposit box.  Measured against
-   the loop that reloaded label and properties at every step (MI355X, kernel time):
-   packed media, isotropic source, 71x64x53, 3e6 photons 169 -> 113 ms; layered 200^3,
-   1e7 photons 151 -> 122 ms; 60^3 pencil beam, 3e5 photons 7.2 -> 6.0 ms; batch of 16
-   48^3 instances 867 -> 764 ms; the 60^3 sphere at 1e8 photons, which the grid
-   atomics bound, 423 -> 421 ms. */
+   every branch), then the waits for the label and the grid atomic behind it; a call too
+   small to fill the chip is bound by its longest photon, ~1e4 steps of ~1 us each.  So
+   the state is updated in place under selects (K_PIN), a run's options sit in one
+   scalar register (features), boundary codes in another, rare branches share one test,
+   the label and the properties are read only where the voxel changes, the energy
+   tallies are registers, which leaves their LDS to the deposit box, and thinned-out
+   waves merge (hand_over).  A load still in flight where branches meet makes the
+   compiler wait for all of them at the head of the loop, the grid atomics too, so
+   every load is pinned where it is read.
+   Measured (MI355X, kernel time): the loop that reloaded label and properties at every
+   step, this loop, this loop with the hand-over and the pinned loads:
+     packed media, isotropic source, 71x64x53, 3e6 photons     169, 113, 111 ms
+     layered 200^3, pencil beam, 1e7 photons                   151, 122, 116 ms
+     60^3 cube, pencil beam, 3e5 photons                       7.2, 6.0, 4.5 ms
+     60^3 sphere, 2e4 photons with records, parity arithmetic  18.0, 16.2, 12.1 ms
+     four 96^3 sources and detectors, parity arithmetic        82, 66, 61 ms
+     batch of 16 48^3 instances                                867, 764, 740 ms
+     60^3 sphere, pencil beam, 1e8 photons (grid atomics)      423, 420, 420 ms */
 /* Transport this lane's photons until its share (fixed map) or its
    workgroup's pool (run-time hand-out) is exhausted.  The photon state starts
    fresh; the RNG, the LDS tables and the lane's scratch come in, and the
    lane's pending grid deposits are flushed before returning. */
 template <bool SAVEDET, bool REFLECT, bool SIMPLE, bool FULL>
-__device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared& sh, Rng& rng, const int idx,
-        float& esc, float& tot) {
+__device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared& sh, Rng& rng, int idx, bool alive,
+        uint32_t thresh) {
+    const uint32_t bcmin = bc_codes(g, 0), bcmax = bc_codes(g, 3), bcdet = bc_detects(g);
+    const float n0 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sh.prop[0].w)));
+    const uint32_t feat0 = features(g);
+    /* parameters of every step in vector registers, where those are to spare: the
+       scalar ones run out, and a reload costs the step its latency */
+    struct {
+        float minenergy, oneoverc0, Rtstep;
+    } hold = {g.minenergy, g.oneoverc0, g.Rtstep};
+    uint64_t mediabase = (uint64_t)g.media;
+
+    if (SIMPLE) {
+        K_PIN(hold.minenergy);
+        K_PIN(hold.oneoverc0);
+        K_PIN(hold.Rtstep);
+        K_PIN(mediabase);
+    }
+
+    uint32_t detsrc = 0, from = 0;
+    DepCache dcache;
+    dcache.a0 = dcache.a1 = 0xFFFFFFFFu;
+    dcache.v0 = dcache.v1 = 0.0;
+    bool moved_on = false;
+    thresh = __builtin_amdgcn_readfirstlane(thresh);
+
+    if (SAVEDET && SIMPLE && __float_as_uint(g.srcparam2.z) < g.nvox) {
+        detsrc = media_at(g, __float_as_uint(g.srcparam2.z)) & K_DET_MASK;
+    }
+
+    /* once, and again after the hand-over for the lanes that run on */
+    for (;;) {
+    bool put = false;
+
+    if (alive) {
     Photon s;
-    s.esc = esc;
-    s.tot = tot;
+    Moving m;
     s.p = make_float4(0.f, 0.f, 0.f, __uint_as_float(0x7FC00000u));
     s.v = make_float4(0.f, 0.f, 0.f, 0.f);
     s.f = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1637,71 +1874,117 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
     s.mediaid = __float_as_uint(g.srcparam2.w);
     s.w0 = 0.f;
     s.Lmove = 0.f;
+    s.esc = s.tot = 0.f;
+    s.sv = 0;
+    m.wre = m.wim = m.pathlen = m.n1 = 0.f;
+    m.isdet = m.detvox = m.launchflag = m.lin = 0;
+    m.relaunch = true;
+    m.testint = false;
+
+    if (FULL && (feat0 & kfSvmc)) {
+        s.sn = sh.pp + g.svoff;
+    }
+
+    if (moved_on) {
+        hand_copy<false>(sh, from, s, rng, idx, m);
+    } else if (g.genergy) {
+        s.esc = g.genergy[idx * 2];
+        s.tot = g.genergy[idx * 2 + 1];
+    }
+
+    /* no load is pending when the loop begins (as in getprop) */
+    pin_photon(s, rng);
+    K_PIN(idx);
+    K_PIN(m.isdet);
+    K_PIN(m.detvox);
+    K_PIN(m.launchflag);
+    K_PIN(m.lin);
+    K_PIN(m.pathlen);
+    K_PIN(m.n1);
+    K_PIN(m.wre);
+    K_PIN(m.wim);
 
     /* the detector flag in effect: the voxel's own, except after a reflection, where
        the reference keeps what the step found beyond the face until the photon's next
        step inside the voxel; detvox is the voxel's own */
-    uint32_t isdet = 0, detvox = 0, launchflag = 0;
-    float pathlen = 0.f, n1 = 0.f;
-    bool relaunch = true;
+    uint32_t isdet = m.isdet, detvox = m.detvox, launchflag = m.launchflag;
+    float pathlen = m.pathlen, n1 = m.n1;
+    bool relaunch = m.relaunch;
     /* linear index of the integer position.  It is idx1d's except after a reflection,
        when idx1d is restored while the position keeps the reflected face's index for
        one step (at a face on the voxel's far side the next voxel's); a deposit then
        goes by idx1d alone, past the box */
-    uint32_t lin = 0;
-    const uint32_t feat0 = features(g);
-    uint32_t detsrc = 0;
-
-    if (SAVEDET && SIMPLE && __float_as_uint(g.srcparam2.z) < g.nvox) {
-        detsrc = media_at(g, __float_as_uint(g.srcparam2.z)) & K_DET_MASK;
-    }
-
-    const uint32_t bcmin = bc_codes(g, 0), bcmax = bc_codes(g, 3), bcdet = bc_detects(g);
-    const float n0 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sh.prop[0].w)));
-    DepCache dcache;
-    dcache.a0 = dcache.a1 = 0xFFFFFFFFu;
-    dcache.v0 = dcache.v1 = 0.0;
+    uint32_t lin = m.lin;
     /* RF forward: the complex photon weight; its value at the last voxel exit is
        read only at exits and sits in the lane scratch at rfoff (real, imaginary) */
     struct {
         float wre, wim;
-    } rf = {0.f, 0.f};
+    } rf = {m.wre, m.wim};
     /* split voxels: test the plane on this step (cleared once the photon crossed
        it, set by a scattering event, a voxel change or some relaunches), and
        whether the step ended on it (src/mcx_core.cl:2342-2343) */
-    bool testint = false, hitintf = false;
-    s.sv = 0;
-
-    if (FULL && g.svmc) {
-        s.sn = sh.pp + g.svoff;
-        s.sn[0] = s.sn[1] = s.sn[2] = s.sn[3] = 0.f;
-    }
-    /* move-only trajectories: the lane's run ends when a photon moves into the
-       background without being relaunched */
-    bool moveend = false;
+    bool testint = m.testint, hitintf = false;
 
     for (;;) {
-        if (relaunch) {
+        /* the wave has thinned out: its lanes move on together with the workgroup's others */
+        const uint64_t live = __ballot(true);
+        bool ended = false;   /* one exit from the loop */
+
+        if ((uint32_t)__popcll(live) <= thresh) {
+            m.wre = rf.wre;
+            m.wim = rf.wim;
+            m.pathlen = pathlen;
+            m.n1 = n1;
+            m.isdet = isdet;
+            m.detvox = detvox;
+            m.launchflag = launchflag;
+            m.lin = lin;
+            m.relaunch = relaunch;
+            m.testint = testint;
+            hand_copy<true>(sh, hand_slot(threadIdx.x >> 6,
+                                          (uint32_t)__popcll(live & ((1ull << (threadIdx.x & 63u)) - 1ull))), s, rng,
+                            idx, m);
+            put = true;
+            ended = true;
+        } else if (relaunch) {
             if (launch_photon<SAVEDET, SIMPLE, FULL>(g, sh, s, rng, idx, launchflag, feat0)) {
-                break;
+                if (g.genergy) {
+                    g.genergy[idx * 2] = s.esc;
+                    g.genergy[idx * 2 + 1] = s.tot;
+                } else {
+                    atomicAdd(sh.energy, (double)s.esc);
+                    atomicAdd(sh.energy + 1, (double)s.tot);
+                }
+
+                ended = true;
+            } else {
+                isdet = SAVEDET ? s.mediaid & K_DET_MASK : 0u;
+                s.mediaid &= K_MED_MASK;
+                n1 = s.prop.w;
+
+                if (SAVEDET) {
+                    /* a source's own label carries no detector flag: the volume's has it */
+                    detvox = SIMPLE ? detsrc : (s.idx1d < g.nvox ? media_at(g, s.idx1d) & K_DET_MASK : 0u);
+                }
+
+                if (!SIMPLE) {
+                    pin_photon(s, rng);
+                    K_PIN(isdet);
+                    K_PIN(detvox);
+                }
+
+                lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+                relaunch = false;
+
+                if (FULL && (feat0 & kfRf)) {
+                    rf.wre = sh.pp[g.rfoff] = s.p.w;
+                    rf.wim = sh.pp[g.rfoff + 1] = 0.f;
+                }
             }
+        }
 
-            isdet = s.mediaid & K_DET_MASK;
-            s.mediaid &= K_MED_MASK;
-            n1 = s.prop.w;
-
-            if (SAVEDET) {
-                /* a source's own label carries no detector flag: the volume's has it */
-                detvox = SIMPLE ? detsrc : (s.idx1d < g.nvox ? media_at(g, s.idx1d) & K_DET_MASK : 0u);
-            }
-
-            lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
-            relaunch = false;
-
-            if (FULL && (feat0 & kfRf)) {
-                rf.wre = sh.pp[g.rfoff] = s.p.w;
-                rf.wim = sh.pp[g.rfoff + 1] = 0.f;
-            }
+        if (ended) {
+            break;
         }
 
         float4& p = s.p;
@@ -1777,8 +2060,9 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     ksincos(tmp0, &sphi, &cphi);
                 } else {
                 if (SIMPLE || !(ft & kf2D)) {
-                    tmp0 = K_TWO_PI * rng.next();
-                    ksincos(tmp0, &sphi, &cphi);
+                    const float turn = rng.next();
+                    tmp0 = K_TWO_PI * turn;
+                    ksincos_turn(turn, &sphi, &cphi);
                 }
 
                 if (!SIMPLE && (ft & kfPhase)) {
@@ -1824,7 +2108,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                 }
 
                 /* per-medium tallies: a split voxel's current side (src/mcx_core.cl:2502-2540) */
-                const uint32_t tlab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : (s.mediaid & K_MED_MASK);
+                const uint32_t tlab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : s.mediaid;
 
                 if (SAVEDET && tlab > 0) {
                     if (ft & kfCountTally) {
@@ -1918,6 +2202,13 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
             K_PIN(gfac);
         }
 
+        if (SIMPLE) {
+            /* one grid atomic in flight per lane: where the atomics bound the run, more of
+               them queue in the memory system without being served any faster (60^3
+               sphere, 1e8 photons: 432 ms unbounded, 418 ms); elsewhere no cost */
+            asm("s_waitcnt vmcnt(0)" : "+v"(s.prop.y));
+        }
+
         float slen = f.z * s.prop.y * gfac;
         /* the scattering site comes before the face */
         bool stay = !(slen < f.x);
@@ -1971,7 +2262,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         uint32_t lab = 0;
 
         if (in & cross) {
-            lab = media_at(g, s.idx1d);
+            lab = ((const K_GLOBAL uint32_t*)mediabase)[s.idx1d];
         }
 
         if (FULL && (ft & kfRf)) {
@@ -1990,10 +2281,10 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         }
 
         f.x -= slen;
-        f.y += f.z * s.prop.w * g.oneoverc0;
+        f.y += f.z * s.prop.w * hold.oneoverc0;
 
         if (SAVEDET && (ft & kfPathTally)) {
-            const uint32_t plab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : (s.mediaid & K_MED_MASK);
+            const uint32_t plab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : s.mediaid;
 
             if (plab > 0) {
                 atomicAdd(&sh.pp[g.maxmedia * ((ft & kfCountTally) ? 1u : 0u) + plab - 1], f.z);
@@ -2013,7 +2304,13 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         /* the deposit: computed for every lane, most of a wave's lanes deposit in most
            steps */
         float weight = 0.f, weight_im = 0.f;
-        int tshift = gate_of(g, f.y);
+        int tshift = 0;
+
+        if (ft & kfGates) {
+            tshift = (int)floorf((f.y - g.twin0) * hold.Rtstep);
+            tshift = tshift > (int)g.maxgate - 1 ? (int)g.maxgate - 1 : tshift;
+        }
+
         bool deposits = moved & ((ft & kfSave) != 0) & (f.y >= g.twin0) & (f.y < g.twin1);
 
         if (FULL && (ft & kfRf)) {
@@ -2135,10 +2432,6 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
             isdet = 0;
         }
 
-        if (cross & !in) {
-            isdet = ((s.idx1d == K_OUT_MAX ? bcmax : bcmin) >> (8 * face)) & 0xFFu;
-        }
-
         if (FULL && (ft & kfSvmc)) {
             /* split voxels (src/mcx_core.cl:2937-2949): a new voxel brings its own
                plane and side; a plane crossing moves the photon to the other side */
@@ -2159,13 +2452,12 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
            or the plane, unless it can reflect there (src/mcx_core.cl:2959-2966) */
         const bool svexit = FULL && (ft & kfSvmc) && (cross || hitintf) && !K_SV_ISUPPER(s.sv) &&
                             !K_SV_LOWER(s.sv) && (!g.doreflect || n1 == n0);
-        const uint32_t code = isdet & 0xFu;
         /* the index the photon comes from; the properties become the new voxel's (a
            reflection reads the old ones again) */
         const float nold = n1;
 
         if (cross && !(FULL && (ft & kfSvmc))) {
-            s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+            s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
         }
 
         n1 = s.prop.w;
@@ -2176,13 +2468,12 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
         }
 
 #endif
-        const bool ends = ((s.mediaid == 0) & ((code == kAbsorb) | (code == kCyclic) | ((code == kReflect) & (nold == n0)))) |
-                          svexit | !(f.y <= g.twin1);
-        const bool mirror = code == kMirror;
-        bool rare = ends | (fabsf(p.w) < g.minenergy);
+        /* everything rare behind one test: a photon outside or in background, out of
+           time, of low weight, or at a change of index */
+        bool rare = (s.mediaid == 0) | svexit | !(f.y <= g.twin1) | (fabsf(p.w) < hold.minenergy);
 
         if (REFLECT) {
-            rare = rare | mirror | (nold != n1) | (FULL && hitintf) | (FULL && (ft & kfMoveOnly));
+            rare = rare | (nold != n1) | (FULL && hitintf) | (FULL && (ft & kfMoveOnly));
         }
 
         if (!rare) {
@@ -2192,6 +2483,15 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
 
             continue;
         }
+
+        if (cross & !in) {
+            isdet = ((s.idx1d == K_OUT_MAX ? bcmax : bcmin) >> (8 * face)) & 0xFFu;
+        }
+
+        const uint32_t code = isdet & 0xFu;
+        const bool mirror = code == kMirror;
+        const bool ends = ((s.mediaid == 0) & ((code == kAbsorb) | (code == kCyclic) | ((code == kReflect) & (nold == n0)))) |
+                          svexit | !(f.y <= g.twin1);
 
         if (ends) {
             bool wrapped = false;
@@ -2218,13 +2518,14 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     isdet = s.mediaid & K_DET_MASK;
                     detvox = isdet;
                     s.mediaid &= K_MED_MASK;
+                    K_PIN(isdet);
                     lin = s.idx1d;
                     /* the next step still compares with the index of the voxel left here,
                        as in the reference */
                     n1 = nold;
 
                     if (!(FULL && (ft & kfSvmc))) {
-                        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+                        s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
                     }
 
                     wrapped = true;
@@ -2337,7 +2638,7 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
                     lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
 
                     if (!(FULL && (ft & kfSvmc))) {
-                        s.prop = getprop<FULL>(g, sh, s.mediaid, s.idx1d, ft);
+                        s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
                     } else {
                         /* the side of the plane the reflected photon lands on; label 0
                            there ends it (src/mcx_core.cl:3221-3243) */
@@ -2359,7 +2660,6 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
             if (FULL && (ft & kfMoveOnly) && (s.mediaid == 0 || s.idx1d == K_OUT_MIN || s.idx1d == K_OUT_MAX)) {
                 /* move-only trajectories (debug flag T, src/mcx_core.cl:3287-3291): the
                    lane's whole run ends here, without its energy write-back */
-                moveend = true;
                 break;
             }
         }
@@ -2370,11 +2670,31 @@ __device__ __forceinline__ bool transport_lane(const MCXKParam& g, const Shared&
             detvox = (cross & !reflected) ? (isdet & K_DET_MASK) : detvox;
         }
     }
+    }
+
+    if (thresh == 0) {
+        break;
+    }
+
+    alive = hand_over(sh, put, rng, from);
+    moved_on = true;
+    thresh = 0;
+    asm("" : "+s"(thresh));   /* one copy of the step loop for both */
+    }
 
     depcache_flush(g, sh, dcache);
-    esc = s.esc;
-    tot = s.tot;
-    return !moveend;
+}
+
+/* Whether this lane draws photons when the workgroup has n of them.  Fewer photons than
+   lanes are spread evenly over just the waves they fill, at least one per SIMD: a wave
+   of few lanes takes fewer of the branches, and waves without any issue nothing.  With
+   no more waves than the hand-over would leave there is no hand-over. */
+__device__ __forceinline__ bool spread_lane(uint32_t n, uint32_t& thresh) {
+    const uint32_t nwave = blockDim.x >> 6, least = (nwave + 3) >> 2;
+    uint32_t waves = (n + 63u) >> 6;
+    waves = waves < least ? least : (waves < nwave ? waves : nwave);
+    thresh = waves > least ? thresh : 0u;
+    return (threadIdx.x >> 6) < waves && (threadIdx.x & 63u) < (n + waves - 1) / waves;
 }
 
 /* The fast build runs one workgroup of bound/64 waves per CU, so the instances that
@@ -2391,18 +2711,23 @@ template <bool SAVEDET, bool REFLECT, bool SIMPLE, bool FULL>
 __global__ void __launch_bounds__(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL))
 MCX_KATTR(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) transport_kernel(const MCXKParam g) {
     extern __shared__ float4 lds[];
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    const int idx = blockIdx.x * g.blocklanes + threadIdx.x;
     const uint32_t pplen = g.pplen;
     __shared__ uint32_t pool[2];
+    __shared__ uint32_t wlive[16];
+    uint32_t thresh = (g.hand && blockDim.x > 64) ? MCX_HAND_LANES : 0u;
     Shared sh;
     /* the parameter block is the kernel's only argument: the kernarg segment starts with it */
     sh.kp = (KParamPtr)__builtin_amdgcn_kernarg_segment_ptr();
     sh.pool = pool;
+    sh.wlive = wlive;
+    sh.energy = NULL;
+    sh.hand = g.hand + (size_t)blockIdx.x * (blockDim.x >> 2) * (MCX_HAND_WORDS + pplen);
     sh.prop = lds;
     sh.invcdf = (float*)(lds + g.medianum);
     sh.box = (BoxCell*)(sh.invcdf + ((g.nphase + 3) & ~3u));
     float* ppbase = (float*)(sh.box + g.box_cells);
-    sh.repoff = (size_t)(idx & (int)(g.nrep - 1)) * g.fieldlen;
+    sh.repoff = (size_t)(blockIdx.x & (g.nrep - 1)) * g.fieldlen;
 
     for (uint32_t i = threadIdx.x; i < g.medianum; i += blockDim.x) {
         sh.prop[i] = g.prop[i];
@@ -2436,26 +2761,28 @@ MCX_KATTR(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) transport_kernel(const MCX
 
     __syncthreads();
 
-    /* lanes without photons skip the transport loop but still join the box flush */
-    const bool active = g.dynamic ? (uint32_t)idx < g.nthread :
+    /* lanes without photons skip the transport loop but still join the hand-over and the
+       box flush */
+    bool active = (uint32_t)idx < g.nthread;
+
+    if (g.dynamic) {
+        active = spread_lane(pool[1], thresh) && active;
+    } else {
+        active = threadIdx.x < g.blocklanes &&
                         !((uint32_t)idx >= g.threadphoton * g.nthread + (uint32_t)g.oddphoton ||
                           (uint32_t)idx >= g.nthread);
-    /* the tail workgroup may hold lanes past nthread: they read nothing */
-    const uint32_t sidx = (uint32_t)idx < g.nthread ? (uint32_t)idx : 0u;
-    float esc = g.genergy[sidx * 2], tot = g.genergy[sidx * 2 + 1];
+    }
+
+    /* lanes that run nothing read the first lane's stream */
+    const uint32_t sidx = active ? (uint32_t)idx : 0u;
     Rng rng;
     rng.s0 = (uint64_t)g.nseed[sidx * 4] << 32 | g.nseed[sidx * 4 + 1];
     rng.s1 = (uint64_t)g.nseed[sidx * 4 + 2] << 32 | g.nseed[sidx * 4 + 3];
-
-    if (active && transport_lane<SAVEDET, REFLECT, SIMPLE, FULL>(g, sh, rng, idx, esc, tot)) {
-        g.genergy[idx * 2] = esc;
-        g.genergy[idx * 2 + 1] = tot;
-    }
+    transport_lane<SAVEDET, REFLECT, SIMPLE, FULL>(g, sh, rng, idx, active, thresh);
 
     if (g.box_cells) {
         /* flush the workgroup's private box into its replica of the global grid */
         __syncthreads();
-        const size_t boff = (size_t)(blockIdx.x & (g.nrep - 1)) * g.fieldlen;
 
         for (uint32_t i = threadIdx.x; i < g.box_cells; i += blockDim.x) {
             double val = (double)sh.box[i];
@@ -2467,19 +2794,10 @@ MCX_KATTR(MCX_KBOUND(SAVEDET, REFLECT, SIMPLE, FULL)) transport_kernel(const MCX
                 uint32_t z = r % g.box_nz, gate = r / g.box_nz;
                 uint32_t vox = (g.box_z0 + z) * g.dimxy + (g.box_y0 + y) * g.dimx + (g.box_x0 + x);
                 gate = (gate < g.box_ng) ? gate : gate - g.box_ng + g.box_imgate;
-                grid_add(g, boff + vox + gate * g.nvox, val);
+                grid_add(g, sh.repoff + vox + gate * g.nvox, val);
             }
         }
     }
-}
-
-/* sum of a double over the 64 lanes of a wave (result in every lane) */
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) {
-        v += __shfl_xor(v, off, 64);
-    }
-
-    return v;
 }
 
 /* Batched transport: many simulations in one persistent launch.
@@ -2491,13 +2809,14 @@ __device__ __forceinline__ double wave_sum(double v) {
    instance with photons left, and moves on when that one is drained; once its
    own list is drained it helps the others.  So an XCD's L2 holds few volumes
    and grids at a time.  On each instance a workgroup stages the tables in LDS,
-   runs its lanes until the counter is exhausted, reduces the launched/escaped
-   weight per wave into the instance's energy tally and flushes its deposit
+   runs its lanes until the counter is exhausted, sums the launched/escaped
+   weight in LDS and adds it to the instance's energy tally, and flushes its deposit
    box.  Lanes keep their RNG streams across instances and write them back at
    the end, so the next launch continues them.  With cost != NULL the
    workgroup's wall-clock time per instance is summed per instance (the
    scheduler's cost probe).
 
+   hand: the workgroups' hand-over slots, handwords words per lane moved.
    state: 2*nqueue words {head, end} of the lists in qlist, then 2 words
    {next photon, end} per instance. */
 template <bool REFLECT>
@@ -2505,9 +2824,12 @@ template <bool REFLECT>
    would take 140 and three waves) */
 __global__ void __launch_bounds__(MCX_BATCH_BLOCK_MAX) __attribute__((amdgpu_waves_per_eu(4))) batch_kernel(const MCXKParam* __restrict__ prm,
         const uint32_t* __restrict__ qlist, const uint32_t nqueue, uint32_t* __restrict__ state,
-        uint32_t* __restrict__ nseed, double* __restrict__ energy, unsigned long long* __restrict__ cost) {
+        uint32_t* __restrict__ nseed, double* __restrict__ energy, unsigned long long* __restrict__ cost,
+        uint32_t* hand, const uint32_t handwords) {
     extern __shared__ float4 lds[];
     __shared__ uint32_t cur;
+    __shared__ uint32_t wlive[16];
+    __shared__ double tally[2];
     uint32_t* const pools = state + 2 * nqueue;
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
     Rng rng;
@@ -2559,6 +2881,9 @@ __global__ void __launch_bounds__(MCX_BATCH_BLOCK_MAX) __attribute__((amdgpu_wav
         Shared sh;
         sh.kp = (KParamPtr)(prm + inst);
         sh.pool = pools + 2 * inst;
+        sh.wlive = wlive;
+        sh.energy = tally;
+        sh.hand = hand + (size_t)blockIdx.x * (blockDim.x >> 2) * handwords;
         sh.prop = lds;
         sh.invcdf = (float*)(lds + g.medianum);
         sh.box = (BoxCell*)(sh.invcdf + ((g.nphase + 3) & ~3u));
@@ -2581,21 +2906,23 @@ __global__ void __launch_bounds__(MCX_BATCH_BLOCK_MAX) __attribute__((amdgpu_wav
             sh.pp[i] = 0.f;
         }
 
+        if (threadIdx.x < 2) {
+            tally[threadIdx.x] = 0.0;
+        }
+
         __syncthreads();
 
         /* the general path only: with the pencil-beam special path inlined beside
            it the kernel needs more registers and runs fewer waves per SIMD */
-        float lesc = 0.f, ltot = 0.f;
-        transport_lane<false, REFLECT, false, false>(g, sh, rng, lane, lesc, ltot);
-
-        const double esc = wave_sum((double)lesc), tot = wave_sum((double)ltot);
-
-        if ((threadIdx.x & 63) == 0 && tot != 0.0) {
-            atomicAdd(energy + 2 * inst, esc);
-            atomicAdd(energy + 2 * inst + 1, tot);
-        }
+        transport_lane<false, REFLECT, false, false>(g, sh, rng, lane, true,
+                hand && blockDim.x > 64 ? MCX_HAND_LANES : 0u);
 
         __syncthreads();
+
+        if (threadIdx.x == 0 && tally[1] != 0.0) {
+            atomicAdd(energy + 2 * inst, tally[0]);
+            atomicAdd(energy + 2 * inst + 1, tally[1]);
+        }
 
         for (uint32_t i = threadIdx.x; i < g.box_cells; i += blockDim.x) {
             double val = (double)sh.box[i];

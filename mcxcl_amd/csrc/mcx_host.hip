@@ -675,7 +675,26 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
     MCXKParam& g = *gp;
     int reflect = 0;
     size_t nthread = *nthread_io;
-    size_t shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, fast ? 0 : MCX_BOX_BYTES, 1);
+    const unsigned int passes = (unsigned int)(cfg->respin < 0 ? -cfg->respin : (cfg->respin ? cfg->respin : 1));
+    /* lanes of the fixed map that run photons.  At a quarter wave per SIMD or fewer they
+       run in one-wave workgroups spread evenly over the chip, since a wave's step takes
+       as long as the branches its lanes take between them: the two replays of a 48^3
+       Jacobian pair (a few thousand photons) 38 -> 32 ms.  With more lanes the waves of
+       a workgroup can merge as their photons end, which one-wave workgroups cannot:
+       2e4 photons (60^3, sphere) 12.4 ms in 256-lane workgroups, 13.4 ms spread. */
+    const size_t mapped = nthread < cfg->nphoton / passes ? nthread : cfg->nphoton / passes;
+    const bool sparse = !dynamic && !envblock && !(cfg->debuglevel & MCX_DEBUG_RNG) && mapped <= (size_t)ncu * 4 * MCX_HAND_LANES;
+
+    if (sparse) {
+        lblock = 64;
+    }
+
+    size_t shmem = mcx_kparam_setup(cfg, &g, nthread, MCX_LAUNCH_BLOCK, &reflect, fast ? 0 : MCX_BOX_BYTES, 1);
+
+    if (sparse && !fast) {
+        shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, MCX_BOX_BYTES, 1);
+    }
+
     {
         const size_t bound = fast ? (size_t)MCX_FAST_BOUND_FULL(cfg->issavedet != 0, reflect != 0, g.simple != 0,
                                  g.full != 0) : MCX_MAX_BLOCK;
@@ -731,12 +750,20 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
         shmem = mcx_kparam_setup(cfg, &g, nthread, lblock, &reflect, budget, 1);
     }
 
-    size_t nlaunch = (nthread + lblock - 1) / lblock;
     /* respin: |respin| repetitions of nphoton/|respin| photons each, every one on
        fresh seeds drawn further down the same rand() stream
        (src/mcx_host.cpp:1089-1104, :1319-1332) */
-    const unsigned int respin = (unsigned int)(cfg->respin < 0 ? -cfg->respin : (cfg->respin ? cfg->respin : 1));
-    const size_t passphoton = cfg->nphoton / respin;
+    const size_t passphoton = cfg->nphoton / passes;
+    g.blocklanes = (uint32_t)lblock;
+
+    if (sparse) {
+        const size_t even = (mapped + (size_t)ncu * 4 - 1) / ((size_t)ncu * 4);
+        g.blocklanes = (uint32_t)(even ? even : 1);
+    }
+
+    /* workgroups of lanes without photons are not launched */
+    size_t nlaunch = (((cfg->debuglevel & MCX_DEBUG_RNG) ? nthread : mapped) + g.blocklanes - 1) / g.blocklanes;
+    nlaunch = nlaunch ? nlaunch : 1;
 
     /* photon split across the persistent threads (src/mcx_host.cpp:1101-1102).
        A lane counts its photons in a float (as the reference's f.w), exact
@@ -773,6 +800,7 @@ static void mcx_plan_run(Config* cfg, int dev, int ncu, size_t* nthread_io, MCXK
                 MCX_ERROR(-4, "too many photons per workgroup (2^32): use respin to split the run");
             }
 
+            g.blocklanes = (uint32_t)lblock;
             nthread = nlaunch * lblock;
             g.nthread = (uint32_t)nthread;
             g.dynamic = 1;
@@ -890,6 +918,8 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
     uint32_t* dnseed = NULL;
     double* dfield = NULL;
     float* dgenergy = NULL;
+    uint32_t* dhand = NULL;
+    size_t handlen = 0;
     float* ddetrec = NULL;
     uint64_t* ddetseed = NULL;
     float* ddetw = NULL;
@@ -1009,8 +1039,13 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
 
     HIP_TRY(dalloc(bufs, &dfield, fieldlen * g.nrep));
     HIP_TRY(hipMemsetAsync(dfield, 0, fieldlen * g.nrep * sizeof(double), stream));
-    HIP_TRY(dalloc(bufs, &dgenergy, nthread * 2));
+    /* the lanes' energies, then the workgroups' hand-over slots (one allocation: each
+       costs a run tens of microseconds to make and free) */
+    handlen = (lblock > 64 && !g.debugrng) ? nlaunch * (lblock / 4) * (MCX_HAND_WORDS + g.pplen) : 0;
+    HIP_TRY(dalloc(bufs, &dgenergy, nthread * 2 + handlen));
     HIP_TRY(hipMemsetAsync(dgenergy, 0, nthread * 2 * sizeof(float), stream));
+    dhand = handlen ? (uint32_t*)(dgenergy + nthread * 2) : NULL;
+
     HIP_TRY(dalloc(bufs, &ddetcount, 1));
     HIP_TRY(hipMemsetAsync(ddetcount, 0, sizeof(uint32_t), stream));
 
@@ -1076,6 +1111,7 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
     g.nseed = dnseed;
     g.field = dfield;
     g.genergy = dgenergy;
+    g.hand = dhand;
     g.detrec = ddetrec;
     g.detseed = ddetseed;
     g.detcount = ddetcount;
