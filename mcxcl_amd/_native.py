@@ -10,6 +10,9 @@ The ctypes ``Config`` structure is laid out from the offsets the library reports
 
 import ctypes
 import os
+import weakref
+
+import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIBPATH = os.path.join(_HERE, "lib", "libmcxhip.so")
@@ -26,6 +29,7 @@ libc.malloc.restype = ctypes.c_void_p
 libc.malloc.argtypes = [ctypes.c_size_t]
 libc.calloc.restype = ctypes.c_void_p
 libc.calloc.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+libc.madvise.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
 libc.free.restype = None
 libc.free.argtypes = [ctypes.c_void_p]
 
@@ -243,11 +247,23 @@ def last_error():
     return msg.decode(errors="replace") if msg else ""
 
 
+def adopt(ptr, ctype, n):
+    """A numpy array over n ctype values of C-allocated memory, freed with the array's
+    last view: the caller drops its own pointer."""
+    buf = (ctype * n).from_address(ptr)
+    weakref.finalize(buf, libc.free, ptr).atexit = False
+    return np.ctypeslib.as_array(buf)
+
+
 def cmalloc(nbytes, zero=True):
     """Allocate with the C allocator so mcx_clearcfg can free it."""
     ptr = libc.calloc(max(1, nbytes), 1) if zero else libc.malloc(max(1, nbytes))
     if not ptr:
         raise MemoryError("malloc(%d) failed" % nbytes)
+    huge = 2 << 20
+    first, last = -(-ptr // huge) * huge, (ptr + nbytes) // huge * huge
+    if last > first:
+        libc.madvise(first, last - first, 14)   # MADV_HUGEPAGE: a fault every 2 MB, not every 4 KB
     return ptr
 
 

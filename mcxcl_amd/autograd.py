@@ -44,6 +44,14 @@ def _as_numpy(t):
     return t.detach().to("cpu", torch.float32).contiguous().numpy()
 
 
+def _media(mua, mus):
+    """[2, Nx, Ny, Nz] in the library's order (mua, mus interleaved, x fastest), so that the
+    runs that share it do not reorder it each"""
+    mm = np.empty((2,) + mua.shape, np.float32, order="F")
+    mm[0], mm[1] = mua, mus
+    return mm
+
+
 def _signal_index(detword, ndet, nsrc):
     """flat (source, detector) index of each detected photon from its detid word"""
     word = detword.astype(np.int64)
@@ -66,7 +74,7 @@ class DetectorSignals(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, mua, mus, cfg):
-        mm = np.stack([_as_numpy(mua), _as_numpy(mus)])
+        mm = _media(_as_numpy(mua), _as_numpy(mus))
         nsrc = _nsrc(cfg)
         run_cfg = dict(cfg, muamus=mm, issavedet=1, issaveseed=1, savedetweight=1, issave2pt=0,
                        savedetflag=cfg.get("savedetflag", "DP"))
@@ -98,18 +106,29 @@ class DetectorSignals(torch.autograd.Function):
         # fold the upstream gradient into the replay weights: one replay of all
         # detected photons then deposits sum g_sd J_sd directly (replaydet 0)
         wg = (detw.astype(np.float64) * g[idx]).astype(np.float32)
-        rep = dict(run_cfg, seed=seeds, detphotons=detp, replayweight=wg, replaydet=0, rawfield=1,
+        rep = dict(run_cfg, seed=seeds, detphotons=detp, replayweight=wg, replaydet=0, rawfield=1, rawonly=1,
                    issaveseed=0, savedetweight=0, issave2pt=1)
         unit = float(run_cfg.get("unitinmm", 1.0))
-        gJ = _run(dict(rep, outputtype="jacobian"))["flux64"].sum(-1).reshape(shape) * unit
-        gW = _run(dict(rep, outputtype="wp"))["flux64"].sum(-1).reshape(shape)
+
+        def replay(outputtype):
+            f = _run(dict(rep, outputtype=outputtype))["flux64"]
+            return (f[..., 0] if f.shape[-1] == 1 else f.sum(-1)).reshape(shape, order="F")
+
+        def tensor(a):
+            # in memory order (x fastest), converted before the transfer
+            return torch.as_tensor(np.asarray(a.T, np.float32), device=grad_s.device).permute(2, 1, 0)
+
         # J holds path lengths in grid units; per-mm derivatives carry unitinmm
-        mus = ctx.mus.astype(np.float64)
-        with np.errstate(divide="ignore", invalid="ignore"):
-            gmus = np.where(mus > 0, gW / mus, 0.0) - gJ
-        grad_mua = torch.as_tensor(-gJ, dtype=torch.float32, device=grad_s.device)
-        grad_mus = torch.as_tensor(gmus, dtype=torch.float32, device=grad_s.device)
-        return grad_mua, grad_mus, None
+        gJ = replay("jacobian") * unit
+        grad_mus = None
+        if ctx.needs_input_grad[1]:
+            # the second replay only where mus is differentiated
+            gW = replay("wp")
+            mus = ctx.mus.astype(np.float64)
+            with np.errstate(divide="ignore", invalid="ignore"):
+                gmus = np.where(mus > 0, gW / mus, 0.0) - gJ
+            grad_mus = tensor(gmus)
+        return tensor(-gJ), grad_mus, None
 
 
 def detector_signals(mua, mus, cfg):
@@ -133,7 +152,7 @@ def signal_jacobians(mua, mus, cfg):
     C-contiguous."""
     mua = np.ascontiguousarray(mua, dtype=np.float32)
     mus = np.ascontiguousarray(mus, dtype=np.float32)
-    mm = np.stack([mua, mus])
+    mm = _media(mua, mus)
     nsrc = _nsrc(cfg)
     ndet = np.atleast_2d(np.asarray(cfg["detpos"])).shape[0]
     run_cfg = dict(cfg, muamus=mm, issavedet=1, issaveseed=1, savedetweight=1, issave2pt=0,

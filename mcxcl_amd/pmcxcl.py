@@ -48,9 +48,12 @@ def _set_vec(dst, values, n):
 
 def _carray(arr, dtype):
     """Copy a numpy array into C-allocated memory (freed by mcx_clearcfg)."""
-    a = np.ascontiguousarray(arr, dtype=dtype)
-    ptr = _native.cmalloc(a.nbytes)
-    ctypes.memmove(ptr, a.ctypes.data, a.nbytes)
+    a = np.asarray(arr)
+    n = max(1, a.size)
+    ptr = _native.cmalloc(n * np.dtype(dtype).itemsize)
+    buf = (ctypes.c_char * (n * np.dtype(dtype).itemsize)).from_address(ptr)
+    # converted on the way in, in one pass
+    np.copyto(np.frombuffer(buf, dtype=dtype)[:a.size].reshape(a.shape), a, casting="unsafe")
     return ptr
 
 
@@ -121,7 +124,7 @@ def _parse_volume(user, c):
     flat = np.asfortranarray(vol).ravel(order="F")
     flat = flat.view(np.uint8).astype(np.uint32) if flat.dtype == np.int8 else flat
     flat = flat.view(np.uint16).astype(np.uint32) if flat.dtype == np.int16 else flat
-    c.vol = _carray(flat.astype(np.uint32), np.uint32)
+    c.vol = _carray(flat, np.uint32)
 
 
 def _parse_srcvec(user, c, key):
@@ -368,8 +371,10 @@ class PreparedConfig:
             self.detw = np.zeros(max(1, int(self.c.maxdetphoton)), dtype=np.float32)
             self.c.exportdetweight = self.detw.ctypes.data
 
-    def collect(self):
-        out = _collect(self.c, self.user, self.ngate, self.ndet, self.nsrc)
+    def collect(self, adopt=False):
+        """the outputs; with adopt their arrays take over the C memory instead of copying it,
+        so a second collect finds none"""
+        out = _collect(self.c, self.user, self.ngate, self.ndet, self.nsrc, adopt)
         if self.detw is not None:
             out["detw"] = self.detw[:self.c.detectedcount].copy()
         dims = [self.c.dim.x, self.c.dim.y, self.c.dim.z, -1]
@@ -417,12 +422,13 @@ def run(cfg=None, **kwargs):
     skipping the normalised float32 copy of large replay grids)."""
     with prepare(cfg, **kwargs) as pc:
         c = pc.c
-        if c.issave2pt and not ((pc.user.get("rawfield") or pc.user.get("rawfield32")) and pc.user.get("rawonly")):
+        if c.issave2pt and (pc.user.get("rawfield") or pc.user.get("rawfield32")) and not pc.user.get("rawonly"):
+            # beside the raw grids the normalised field is only made for a caller that passes its array
             c.exportfield = _native.cmalloc(4 * pc.fieldlen)
         rc = lib.mcx_try_run_simulation(ctypes.byref(c))
         if rc:
             raise RuntimeError("MCX terminated due to an exception: " + _native.last_error())
-        return pc.collect()
+        return pc.collect(adopt=True)
 
 
 class Batch:
@@ -504,8 +510,16 @@ def _is_complex(c):
         (c.omega > 0 and c.seed != SEED_FROM_FILE)
 
 
-def _collect(c, user, ngate, ndet, nsrc):
+def _collect(c, user, ngate, ndet, nsrc, adopt=False):
     out = {}
+
+    def take(field, ctype, n):
+        ptr = getattr(c, field)
+        if adopt:
+            setattr(c, field, None)
+            return _native.adopt(ptr, ctype, n)
+        return np.ctypeslib.as_array((ctype * n).from_address(ptr)).copy()
+
     reclen = lib.mcx_detreclen(ctypes.byref(c))
     n = c.detectedcount
     if c.issaveseed and c.seeddata and c.issavedet:
@@ -515,7 +529,7 @@ def _collect(c, user, ngate, ndet, nsrc):
         vol = np.ctypeslib.as_array((ctypes.c_uint32 * (c.dim.x * c.dim.y * c.dim.z)).from_address(c.vol)).copy()
         out["vol"] = vol.reshape((c.dim.x, c.dim.y, c.dim.z), order="F")
     if c.issavedet and n > 0 and reclen > 0:
-        det = np.ctypeslib.as_array((ctypes.c_float * (reclen * n)).from_address(c.exportdetected)).copy()
+        det = take("exportdetected", ctypes.c_float, reclen * n)
         out["detp"] = np.asfortranarray(det.reshape(n, reclen).T)
     if (c.debuglevel & (MCX_DEBUG_MOVE | MCX_DEBUG_MOVE_ONLY)) and c.exportdebugdata and c.debugdatalen:
         # trajectory positions [6, N]: photon id (uint32 bits), x, y, z, weight, source id
@@ -533,17 +547,17 @@ def _collect(c, user, ngate, ndet, nsrc):
             # RF replay: real and imaginary halves along the last axis (src/pmcxcl.cpp:1339-1345)
             dims += [1] * (5 - len(dims)) + [nsrc * nrf]
         total = int(np.prod(dims))
-        flux = np.ctypeslib.as_array((ctypes.c_float * total).from_address(c.exportfield)).copy()
+        flux = take("exportfield", ctypes.c_float, total)
         flux = flux.reshape(dims, order="F")
         if c.issaveref:
-            volmask = np.ctypeslib.as_array(
-                (ctypes.c_uint32 * (c.dim.x * c.dim.y * c.dim.z)).from_address(c.vol)).copy()
-            inside = (volmask & 0x7FFFFFFF).reshape((c.dim.x, c.dim.y, c.dim.z), order="F") > 0
-            fl = flux.reshape((c.dim.x, c.dim.y, c.dim.z, -1), order="F")
-            dref = np.where(inside[..., None], 0.0, -fl).astype(np.float32)
-            fl[~inside] = 0.0
-            out["dref"] = dref.reshape(dims, order="F")
-            flux = fl.reshape(dims, order="F")
+            # in memory order, touching the voxels outside the domain only
+            words = np.ctypeslib.as_array((ctypes.c_uint32 * (c.dim.x * c.dim.y * c.dim.z)).from_address(c.vol))
+            outside = np.flatnonzero((words == 0) | (words == 0x80000000))
+            fl = flux.reshape(-1, order="F").reshape(-1, words.size)
+            dref = np.zeros(fl.shape, np.float32)
+            dref[:, outside] = -fl[:, outside]
+            fl[:, outside] = 0.0
+            out["dref"] = dref.reshape(-1).reshape(dims, order="F")
         if c.omega > 0 and c.seed != SEED_FROM_FILE:
             # RF forward: complex fluence, real half + 1j * imaginary half (src/pmcxcl.cpp:1387-1408);
             # with pooled sources one complex field per source along the last axis
@@ -562,7 +576,7 @@ def _collect(c, user, ngate, ndet, nsrc):
         keys = ADJOINT_KEYS.get(ot, ())
         # RF forward: complex64, the imaginary blocks after the real ones (src/pmcxcl.cpp:1459-1485)
         nrf = 2 if (c.omega > 0 and c.seed != SEED_FROM_FILE) else 1
-        buf = np.ctypeslib.as_array((ctypes.c_float * (adjlen * len(keys) * nrf)).from_address(c.exportjacob)).copy()
+        buf = take("exportjacob", ctypes.c_float, adjlen * len(keys) * nrf)
         for k, name in enumerate(keys):
             v = buf[k * adjlen:(k + 1) * adjlen]
             if nrf == 2:

@@ -1,0 +1,72 @@
+"""Seeding words across the edges of the generator's runs, result arrays that take over
+the library's memory, and the absorption gradient alone."""
+
+import ctypes
+import gc
+
+import numpy as np
+import pytest
+
+import mcxcl_amd
+from mcxcl_amd import _native, pmcxcl, workloads
+
+
+@pytest.mark.parametrize("n", [1, 30, 31, 34, 1023, 1024, 1025, 2048, 5000])
+def test_seed_words_equal_the_c_library(n):
+    got = np.zeros(n, np.uint32)
+    _native.lib.mcx_host_seed_words(97, n, got.ctypes.data_as(ctypes.POINTER(ctypes.c_uint)))
+    _native.libc.srand(97)
+    assert got.tolist() == [_native.libc.rand() for _ in range(n)]
+
+
+def test_adopted_memory_lives_with_its_last_view():
+    ptr = _native.cmalloc(4 << 20)
+    view = _native.adopt(ptr, ctypes.c_float, 1 << 20).reshape(1024, 1024)[5]
+    view[:] = 7.0
+    gc.collect()
+    _native.cmalloc(4 << 20)
+    assert (view == 7.0).all() and view.flags.writeable
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("raw", [{}, {"rawfield": 1}, {"rawfield32": 1}, {"rawfield": 1, "rawonly": 1}])
+def test_results_outlive_later_runs(raw):
+    """exact: the bit-reproducible arithmetic on a fixed map, grids summed in another order
+    (float64, rounded to float32: 1e-6)"""
+    cfg = workloads.sphere_cube_workload(nphoton=20000, autopilot=0, nthread=2048, nblocksize=64, mathmode=1,
+                                         issavedet=1, issaveseed=1, savedetflag="DSP", **raw)
+    a = mcxcl_amd.run(cfg)
+    kept = {k: v.copy() for k, v in a.items() if isinstance(v, np.ndarray)}
+    with pmcxcl.prepare(cfg) as pc:      # a prepared run collects as often as it is asked
+        if not raw:
+            assert _native.lib.mcx_try_run_simulation(ctypes.byref(pc.c)) == 0
+            one, two = pc.collect(), pc.collect()
+            assert all(np.array_equal(one[k], two[k]) for k in kept)
+    b = mcxcl_amd.run(dict(cfg, seed=1234567))
+    assert all(np.array_equal(a[k], kept[k]) for k in kept)
+    assert ("flux" in a) == (not raw.get("rawonly"))
+    if "flux" in a:
+        assert a["flux"].flags.writeable and not np.array_equal(a["flux"], b["flux"])
+    if raw.get("rawfield"):
+        c = mcxcl_amd.run(dict(cfg, rawonly=0))
+        np.testing.assert_allclose(c["flux64"], a["flux64"], rtol=1e-9, atol=1e-12)
+
+
+@pytest.mark.gpu
+def test_absorption_gradient_alone_equals_the_joint_one():
+    torch = pytest.importorskip("torch")
+    from mcxcl_amd import autograd
+    vol = np.ones((12, 10, 8), np.uint8)
+    cfg = dict(nphoton=20000, vol=vol, prop=[[0, 0, 1, 1], [0.01, 1.0, 0.5, 1.37]], srcpos=[6, 5, 0], srcdir=[0, 0, 1],
+               detpos=[[3, 5, 0, 2], [9, 5, 0, 2]], tstart=0, tend=1e-9, tstep=1e-9, seed=11, mathmode=1,
+               autopilot=0, nthread=1024, nblocksize=64)
+    grads = []
+    for both in (False, True):
+        mua = torch.full(vol.shape, 0.01, requires_grad=True)
+        mus = torch.full(vol.shape, 1.0, requires_grad=both)
+        autograd.detector_signals(mua, mus, cfg).sum().backward()
+        assert (mus.grad is not None) == both
+        grads.append(mua.grad.numpy())
+    # the replay's float64 deposits in another order, rounded to float32
+    np.testing.assert_allclose(grads[0], grads[1], rtol=1e-6, atol=1e-12)
+    assert np.abs(grads[0]).sum() > 0
