@@ -47,6 +47,8 @@ def _as_numpy(t):
 def _media(mua, mus):
     """[2, Nx, Ny, Nz] in the library's order (mua, mus interleaved, x fastest), so that the
     runs that share it do not reorder it each"""
+    if mua.shape != mus.shape:
+        raise ValueError("mua and mus must have the same shape, not %s and %s" % (mua.shape, mus.shape))
     mm = np.empty((2,) + mua.shape, np.float32, order="F")
     mm[0], mm[1] = mua, mus
     return mm

@@ -280,3 +280,17 @@ def test_mus_gradient_on_device_matches_layerwise_finite_differences(monkeypatch
     base = workloads.sphere_cube_workload(nphoton=2000000, tstep=5e-9, mathmode=0)
     for label in (1, 2):
         _assert_mus_scaling(_mus_scaling_check(base, label, 0.1, 500 + 31 * np.arange(8), 2000000))
+
+
+@pytest.mark.parametrize("shape", [(), (4,), (1, 1, 4), (6, 5, 1)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_shapes_that_differ_are_refused(monkeypatch, shape, swap):
+    """no broadcasting between the two property arrays, before anything runs"""
+    monkeypatch.setattr(autograd, "_run", lambda cfg: pytest.fail("ran"))
+    a, b = np.full((6, 5, 4), 0.01, np.float32), np.full(shape, 1.0, np.float32)
+    a, b = (b, a) if swap else (a, b)
+    cfg = {"detpos": [[1, 1, 0, 1]]}
+    with pytest.raises(ValueError, match="same shape"):
+        autograd.detector_signals(torch.from_numpy(a), torch.from_numpy(b), cfg)
+    with pytest.raises(ValueError, match="same shape"):
+        autograd.signal_jacobians(a, b, cfg)
