@@ -129,7 +129,8 @@ class DetectorSignals(torch.autograd.Function):
             mus = ctx.mus.astype(np.float64)
             with np.errstate(divide="ignore", invalid="ignore"):
                 gmus = np.where(mus > 0, gW / mus, 0.0) - gJ
-            grad_mus = tensor(gmus)
+            # C-contiguous, as this gradient always was
+            grad_mus = torch.as_tensor(np.ascontiguousarray(gmus, np.float32), device=grad_s.device)
         return tensor(-gJ), grad_mus, None
 
 

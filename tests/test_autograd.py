@@ -294,3 +294,26 @@ def test_shapes_that_differ_are_refused(monkeypatch, shape, swap):
         autograd.detector_signals(torch.from_numpy(a), torch.from_numpy(b), cfg)
     with pytest.raises(ValueError, match="same shape"):
         autograd.signal_jacobians(a, b, cfg)
+
+
+@pytest.mark.parametrize("shape", [(6, 5, 4), (1, 5, 4), (6, 1, 1)])
+def test_mus_gradient_is_contiguous(monkeypatch, shape):
+    """a caller may flatten it with .view, from a hook or torch.autograd.grad; its values are
+    WP / mus - J of the replays' grids, rounded once to float32"""
+    rng = np.random.default_rng(3)
+    grids = {t: np.asfortranarray(rng.uniform(1, 2, shape + (1,))) for t in ("jacobian", "wp")}
+
+    def run(cfg):
+        if "outputtype" in cfg:
+            return {"flux64": grids[cfg["outputtype"]]}
+        return {"detp": np.ones((2, 3), np.float32), "detw": np.ones(3, np.float32), "seeds": np.zeros((16, 3), np.uint8)}
+
+    monkeypatch.setattr(autograd, "_run", run)
+    mua = torch.full(shape, 0.01, requires_grad=True)
+    mus = torch.from_numpy(rng.uniform(1, 2, shape).astype(np.float32)).requires_grad_()
+    signals = autograd.detector_signals(mua, mus, {"srcpos": [0, 0, 0], "detpos": [[1, 1, 0, 1]]})
+    gmua, gmus = torch.autograd.grad(signals.sum(), [mua, mus])
+    want = grids["wp"][..., 0] / mus.detach().numpy().astype(np.float64) - grids["jacobian"][..., 0]
+    assert gmus.is_contiguous()
+    np.testing.assert_array_equal(gmus.view(-1).numpy(), want.astype(np.float32).ravel())
+    np.testing.assert_array_equal(gmua.numpy(), -grids["jacobian"][..., 0].astype(np.float32))
