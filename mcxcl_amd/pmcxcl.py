@@ -325,7 +325,10 @@ class PreparedConfig:
             self.close()
             raise
         c = self.c
-        self.ngate = int((c.tend - c.tstart) / c.tstep + 0.5)
+        # in single precision, as the library counts them: in double a window of 1.5 gates
+        # rounds the other way, and the library would fill a longer array than this one
+        f32 = np.float32
+        self.ngate = int(float((f32(c.tend) - f32(c.tstart)) / f32(c.tstep)) + 0.5)
         self.nvox = c.dim.x * c.dim.y * c.dim.z
         self.ndet = c.detnum if (c.seed == SEED_FROM_FILE and c.replaydet == -1) else 1
         self.nsrc = (c.extrasrclen + 1) if (c.extrasrclen and c.srcid < 0) else 1

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import mcxcl_amd
+import oracle
 from mcxcl_amd import _native, pmcxcl, workloads
 
 
@@ -70,3 +71,16 @@ def test_absorption_gradient_alone_equals_the_joint_one():
     # the replay's float64 deposits in another order, rounded to float32
     np.testing.assert_allclose(grads[0], grads[1], rtol=1e-6, atol=1e-12)
     assert np.abs(grads[0]).sum() > 0
+
+
+@pytest.mark.parametrize("tend,tstep", [(3e-10, 2e-10), (5e-10, 2e-10), (1e-9, 4e-10), (1.3e-9, 2e-10), (5e-9, 5e-10),
+                                        (5e-9, 1.1e-9)])
+def test_gates_are_counted_as_the_library_does(tend, tstep):
+    """windows of a whole number of gates and a half, where single and double precision round
+    to different counts: the arrays handed to the library hold what it fills"""
+    cfg = workloads.homogeneous_cube_workload(nphoton=100, vol=np.ones((5, 6, 7), np.uint8), srcpos=[2, 2, 0],
+                                              tstart=0, tend=tend, tstep=tstep)
+    out = oracle.run(dict(cfg, autopilot=0, nthread=64, nblocksize=64), nthread=64)
+    with pmcxcl.prepare(dict(cfg, rawfield=1)) as pc:
+        assert pc.raw.size == out["flux64"].size
+    assert out["flux"].shape[3] == out["flux64"].shape[3]
