@@ -225,7 +225,8 @@ struct DevBuf {
 /* huge pages for a large array a result is read back into, so that the copy does not
    take a fault every 4 KB (four 96^3 sources and detectors, 113 MB of adjoint outputs:
    27 ms on 4 KB pages, 12 ms) */
-void* on_huge_pages(void* p, size_t bytes) {
+void* host_result(size_t bytes) {
+    void* p = malloc(bytes ? bytes : 1);
     const uintptr_t huge = (uintptr_t)2 << 20, first = ((uintptr_t)p + huge - 1) / huge * huge,
                     last = ((uintptr_t)p + bytes) / huge * huge;
 
@@ -234,10 +235,6 @@ void* on_huge_pages(void* p, size_t bytes) {
     }
 
     return p;
-}
-
-void* host_result(size_t bytes) {
-    return on_huge_pages(malloc(bytes ? bytes : 1), bytes);
 }
 
 double wall_ms() {
@@ -1474,8 +1471,7 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
         if (wantfloat) {
             /* a caller without a buffer gets the array that was read back */
             newfield = !cfg->exportfield;
-            hfield = newfield ? (float*)on_huge_pages(calloc(fieldlen * 2, sizeof(float)), fieldlen * sizeof(float)) :
-                     (float*)host_result(fieldlen * sizeof(float));
+            hfield = (float*)host_result(fieldlen * sizeof(float));
 
             if (!hfield) {
                 HIP_TRY(hipErrorOutOfMemory);

@@ -84,3 +84,16 @@ def test_gates_are_counted_as_the_library_does(tend, tstep):
     with pmcxcl.prepare(dict(cfg, rawfield=1)) as pc:
         assert pc.raw.size == out["flux64"].size
     assert out["flux"].shape[3] == out["flux64"].shape[3]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("extra", [{}, {"omega": 2 * np.pi * 1e8}, {"tstep": 5e-10}])
+def test_returned_field_holds_no_more_than_itself(extra):
+    """the array that is handed over keeps the block it was read back into: the field's size,
+    up to the allocator's rounding"""
+    _native.libc.malloc_usable_size.restype = ctypes.c_size_t
+    _native.libc.malloc_usable_size.argtypes = [ctypes.c_void_p]
+    cfg = dict(workloads.sphere_cube_workload(nphoton=2000, issavedet=0), **extra)
+    with pmcxcl.prepare(cfg) as pc:
+        assert _native.lib.mcx_try_run_simulation(ctypes.byref(pc.c)) == 0
+        assert _native.libc.malloc_usable_size(pc.c.exportfield) <= 4 * pc.fieldlen + 8192
