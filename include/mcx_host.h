@@ -62,6 +62,11 @@ int mcx_device_count(void);
    RNG streams (src/mcx_host.cpp:696-700, :759-768) */
 void mcx_host_seed_words(unsigned int seed, size_t n, unsigned int* out);
 
+/* the LDS deposit box of a run whose workgroups have boxbytes for it: origin,
+   edges and gates in box[7], all 0 without one.  Host only, for the test suite.
+   Returns 0 or the error id. */
+int mcx_deposit_box(Config* cfg, size_t boxbytes, unsigned int* box);
+
 /* self-checks of the device arithmetic, for the test suite: evaluate the
    kernel's single-precision math (which: 0 exp, 1 log, 2 sin, 3 cos, 4 acos,
    5 rsqrt, 6 divide x[i]/x[i+n], 7 sqrt) in parity mode (mode 1) or fast mode

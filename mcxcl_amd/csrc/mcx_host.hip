@@ -611,23 +611,41 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
 
         /* Under a source wider than that the deposits are as dense as under its middle,
            so the box spans the source and takes the depth that is left, down to
-           MCX_BOX_DEPTH_MIN layers; then it spans what it can.  40x40 planar source on
-           60^3, one gate, 1e7 photons: 37x37x27 at the corner 58.4 ms, 40x40x25 under
-           the source 37.5 ms; 100x100 on 160x160x60, 4e6 photons, 70x70x8: 40.1, 36.8 ms */
+           MCX_BOX_DEPTH_MIN layers; then it spans what it can.  Across a narrow source
+           (a slit) the light spreads as far as it reaches down, so that side keeps the
+           depth's 4/3 at least.  What the grid's depth leaves over goes to the sides.
+           Kernel time of the box at the source's corner, under it as wide as it, this
+           one (one gate):
+             40x40 on 60^3, 5e6 photons, 40x40x23             32.6, 19.1, 19.2 ms
+             40x1 on 60^3, 5e6 photons, 40x1x60 -> 40x35x26   34.2, 58.7, 19.8 ms
+             60x2 on 100^3, 4e6 photons, 60x2x100 -> 60x28x22 48.9, 44.2, 23.7 ms
+             60x4 on 120x120x12, 4e6 photons                  30.0, 20.6, 13.5 ms
+             100x100 on 160x160x60, 3e6 photons, 68x68x8      32.9, 27.7, 27.8 ms */
         if (depth >= 0) {
             const int a = (depth + 1) % 3, b = (depth + 2) % 3;
 
             if (width[a] > (float)edge[a] || width[b] > (float)edge[b]) {
-                float wa = width[a] > 1.f ? (width[a] < (float)dims[a] ? ceilf(width[a]) : (float)dims[a]) : 1.f;
-                float wb = width[b] > 1.f ? (width[b] < (float)dims[b] ? ceilf(width[b]) : (float)dims[b]) : 1.f;
+                const float da = (float)dims[a], db = (float)dims[b], fcells = (float)cells / (float)ng;
+                float wa = fminf(fmaxf(ceilf(width[a]), 1.f), da), wb = fminf(fmaxf(ceilf(width[b]), 1.f), db);
+                const float side = floorf(sqrtf(fcells / (0.75f * fmaxf(wa, wb))));
+                wa = fminf(fmaxf(wa, side), da);
+                wb = fminf(fmaxf(wb, side), db);
                 const float layers = (float)(dims[depth] < MCX_BOX_DEPTH_MIN ? dims[depth] : MCX_BOX_DEPTH_MIN);
-                const float fit = sqrtf((float)cells / ((float)ng * layers * wa * wb));
+                const float fit = sqrtf(fcells / (layers * wa * wb));
                 wa = fit < 1.f ? floorf(wa * fit) : wa;
                 wb = fit < 1.f ? floorf(wb * fit) : wb;
                 edge[a] = wa < 1.f ? 1u : (unsigned int)wa;
                 edge[b] = wb < 1.f ? 1u : (unsigned int)wb;
-                const size_t d = cells / (ng * edge[a] * edge[b]);
-                edge[depth] = d < 1 ? 1u : (d < dims[depth] ? (unsigned int)d : dims[depth]);
+                const size_t deep = cells / (ng * edge[a] * edge[b]);
+                edge[depth] = deep < 1 ? 1u : (deep < dims[depth] ? (unsigned int)deep : dims[depth]);
+                const size_t area = cells / (ng * edge[depth]);
+                const unsigned int square = (unsigned int)sqrtf((float)area);
+                const int n = edge[a] < edge[b] ? a : b, w = a + b - n;
+                edge[w] = edge[w] < square ? (square < dims[w] ? square : dims[w]) : edge[w];
+                const size_t rn = area / edge[w];
+                edge[n] = rn > edge[n] ? (rn < dims[n] ? (unsigned int)rn : dims[n]) : edge[n];
+                const size_t rw = area / edge[n];
+                edge[w] = rw > edge[w] ? (rw < dims[w] ? (unsigned int)rw : dims[w]) : edge[w];
             }
         }
 
@@ -683,6 +701,25 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
     }
 
     return shmem;
+}
+
+/* the deposit box of a run whose workgroups have boxbytes of LDS for it:
+   {x0, y0, z0, nx, ny, nz, gates}, all 0 without one; needs no device */
+extern "C" int mcx_deposit_box(Config* cfg, size_t boxbytes, unsigned int* box) {
+    jmp_buf jb;
+    void* old = mcx_push_errjmp(&jb);
+    int rc = setjmp(jb);
+
+    if (rc == 0) {
+        MCXKParam g;
+        int reflect = 0;
+        (void)mcx_kparam_setup(cfg, &g, 64, 64, &reflect, boxbytes, 1);
+        const unsigned int b[7] = {g.box_x0, g.box_y0, g.box_z0, g.box_nx, g.box_ny, g.box_nz, g.box_ng};
+        memcpy(box, b, sizeof(b));
+    }
+
+    mcx_pop_errjmp(old);
+    return rc;
 }
 
 /* pixels of a pattern source: param1.w x param2.w (pattern), param1.x x
