@@ -67,6 +67,10 @@ void mcx_host_seed_words(unsigned int seed, size_t n, unsigned int* out);
    Returns 0 or the error id. */
 int mcx_deposit_box(Config* cfg, size_t boxbytes, unsigned int* box);
 
+/* 32-bit words of device memory for the hand-over slots of a run of nlaunch
+   workgroups of lblock lanes with pplen words of scratch each; 0: none. */
+size_t mcx_hand_over_words(size_t nlaunch, size_t lblock, size_t pplen);
+
 /* self-checks of the device arithmetic, for the test suite: evaluate the
    kernel's single-precision math (which: 0 exp, 1 log, 2 sin, 3 cos, 4 acos,
    5 rsqrt, 6 divide x[i]/x[i+n], 7 sqrt) in parity mode (mode 1) or fast mode

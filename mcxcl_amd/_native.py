@@ -206,6 +206,8 @@ lib.mcx_list_gpu.restype = ctypes.c_int
 lib.mcx_device_count.restype = ctypes.c_int
 lib.mcx_host_seed_words.argtypes = [ctypes.c_uint, ctypes.c_size_t, ctypes.c_void_p]
 lib.mcx_host_seed_words.restype = None
+lib.mcx_hand_over_words.argtypes = [ctypes.c_size_t] * 3
+lib.mcx_hand_over_words.restype = ctypes.c_size_t
 lib.mcx_deposit_box.argtypes = [ctypes.POINTER(Config), ctypes.c_size_t, ctypes.POINTER(ctypes.c_uint)]
 lib.mcx_device_fpmath.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
                                   ctypes.c_size_t]

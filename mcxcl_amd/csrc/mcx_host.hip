@@ -36,6 +36,7 @@
 #define MCX_BOX_EDGE_MAX 48u
 #define MCX_BOX_DEPTH_MIN 8u   /* layers under an area source, at least */
 #define MCX_BOX_BYTES (32u * 1024u)
+#define MCX_HAND_BYTES ((size_t)1 << 30)   /* hand-over slots of one run, at most */
 #define MCX_LDS_LIMIT (160u * 1024u)
 /* LDS kept back from the fast build's box budget: static LDS and allocation
    granularity */
@@ -703,6 +704,15 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
     return shmem;
 }
 
+/* words of a run's hand-over slots (a quarter of its lanes, each with its scratch), 0 for
+   none.  They only save time, so a map too large for MCX_HAND_BYTES (2e7 lanes with a few
+   record columns) goes without.  60^3 cube, bit-reproducible arithmetic, a photon a lane,
+   without and with them: 4e6 lanes 120, 102 ms */
+extern "C" size_t mcx_hand_over_words(size_t nlaunch, size_t lblock, size_t pplen) {
+    const size_t words = lblock > 64 ? nlaunch * (lblock / 4) * (MCX_HAND_WORDS + pplen) : 0;
+    return words * sizeof(uint32_t) <= MCX_HAND_BYTES ? words : 0;
+}
+
 /* the deposit box of a run whose workgroups have boxbytes of LDS for it:
    {x0, y0, z0, nx, ny, nz, gates}, all 0 without one; needs no device */
 extern "C" int mcx_deposit_box(Config* cfg, size_t boxbytes, unsigned int* box) {
@@ -1036,7 +1046,6 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
     uint32_t* dnseed = NULL;
     double* dfield = NULL;
     float* dgenergy = NULL;
-    uint32_t* dhand = NULL;
     size_t handlen = 0, nactive = 0;
     float* ddetrec = NULL;
     uint64_t* ddetseed = NULL;
@@ -1161,13 +1170,6 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
 
     HIP_TRY(dalloc(bufs, &dfield, fieldlen * g.nrep));
     HIP_TRY(hipMemsetAsync(dfield, 0, fieldlen * g.nrep * sizeof(double), stream));
-    /* the lanes' energies, then the workgroups' hand-over slots (one allocation: each
-       costs a run tens of microseconds to make and free) */
-    handlen = (lblock > 64 && !g.debugrng) ? nlaunch * (lblock / 4) * (MCX_HAND_WORDS + g.pplen) : 0;
-    HIP_TRY(dalloc(bufs, &dgenergy, nactive * 2 + handlen));
-    HIP_TRY(hipMemsetAsync(dgenergy, 0, nactive * 2 * sizeof(float), stream));
-    dhand = handlen ? (uint32_t*)(dgenergy + nactive * 2) : NULL;
-
     HIP_TRY(dalloc(bufs, &ddetcount, 1));
     HIP_TRY(hipMemsetAsync(ddetcount, 0, sizeof(uint32_t), stream));
 
@@ -1232,8 +1234,6 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
     g.replayseed = dreplayseed;
     g.nseed = dnseed;
     g.field = dfield;
-    g.genergy = dgenergy;
-    g.hand = dhand;
     g.detrec = ddetrec;
     g.detseed = ddetseed;
     g.detcount = ddetcount;
@@ -1272,6 +1272,23 @@ extern "C" void mcx_run_simulation(Config* cfg, float* fluence, float* totalener
             HIP_TRY(dalloc(bufs, &draw32, fieldlen));
         }
     }
+
+    /* the lanes' energies, then the workgroups' hand-over slots (one allocation: each
+       costs a run tens of microseconds to make and free), after all that the run cannot do
+       without: with no room left for the slots it goes on without them */
+    handlen = g.debugrng ? 0 : mcx_hand_over_words(nlaunch, lblock, g.pplen);
+    err = dalloc(bufs, &dgenergy, nactive * 2 + handlen);
+
+    if (err != hipSuccess && handlen) {
+        (void)hipGetLastError();
+        handlen = 0;
+        err = dalloc(bufs, &dgenergy, nactive * 2);
+    }
+
+    HIP_TRY(err);
+    HIP_TRY(hipMemsetAsync(dgenergy, 0, nactive * 2 * sizeof(float), stream));
+    g.genergy = dgenergy;
+    g.hand = handlen ? (uint32_t*)(dgenergy + nactive * 2) : NULL;
 
     HIP_TRY(hipStreamSynchronize(stream));
     t0 = wall_ms();

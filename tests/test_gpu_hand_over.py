@@ -189,3 +189,11 @@ def test_batch_workgroups_launch_every_photon(blocksize):
         assert out["stat"]["energytot"] == n
         p = _absorbed(mcxcl_amd.run(dict(cfg, nphoton=200000, mathmode=1)), 200000)
         assert (np.abs(_absorbed(out, n) - p) <= 6 * np.sqrt(p * (1 - p) * (1 / n + 1 / 200000))).all()
+
+
+def test_a_map_of_many_lanes_matches_oracle():
+    """four times the default map's lanes; a short window keeps the oracle quick"""
+    n = 2700000
+    cfg = workloads.sphere_cube_workload(nphoton=n, tend=1e-10, tstep=1e-10, **_DET)
+    cfg = dict(cfg, autopilot=0, nthread=n + 32, nblocksize=64, mathmode=1, rawfield=1)
+    _agree(mcxcl_amd.run(cfg), oracle.run(cfg, nthread=n + 32), ["detp"])

@@ -73,6 +73,16 @@ def test_absorption_gradient_alone_equals_the_joint_one():
     assert np.abs(grads[0]).sum() > 0
 
 
+@pytest.mark.parametrize("scratch", [0, 10, 500])
+def test_hand_over_slots_stay_within_their_bound(scratch):
+    """the default map has them, and no map takes more than 1 GiB for them"""
+    words = _native.lib.mcx_hand_over_words
+    assert words(655360 // 256, 256, scratch) == 655360 // 4 * (42 + scratch)
+    assert words(256, 1024, scratch) == 65536 * (42 + scratch) and words(40000, 64, scratch) == 0
+    for lanes in (1 << 20, 1 << 22, 10 ** 7, 1 << 26, 1 << 30):
+        assert 4 * words(lanes // 256, 256, scratch) <= 1 << 30
+
+
 @pytest.mark.parametrize("tend,tstep", [(3e-10, 2e-10), (5e-10, 2e-10), (1e-9, 4e-10), (1.3e-9, 2e-10), (5e-9, 5e-10),
                                         (5e-9, 1.1e-9)])
 def test_gates_are_counted_as_the_library_does(tend, tstep):
