@@ -22,6 +22,9 @@
    four waves fit in one), and the words a lane moves besides its LDS scratch */
 #define MCX_HAND_LANES 16u
 #define MCX_HAND_WORDS 42u
+/* limit of a float32 deposit-box cell, and the one under area sources (powers of two) */
+#define MCX_BOX_LIMIT 256.f
+#define MCX_BOX_LIMIT_MIN 32.f
 #define MCX_FAST_SIMPLE_BLOCK 1024
 /* waves per SIMD the fast kernels are built for (amdgpu_waves_per_eu caps them) */
 #define MCX_FAST_WAVES 4
@@ -63,6 +66,7 @@ struct MCXKParam {
        (box_imgate = imoff / nvox; 0 when the box holds no imaginary half) */
     uint32_t box_x0, box_y0, box_z0, box_nx, box_ny, box_nz, box_ng, box_cells;
     uint32_t box_imgate;
+    uint32_t box_tight;           /* 1: float32 cells are held within MCX_BOX_LIMIT_MIN, not MCX_BOX_LIMIT */
     uint32_t stokesoff;           /* polarised runs: the Stokes vector's offset in the lane scratch */
     uint32_t rfoff;               /* RF forward: offset of the weight at the last voxel exit (re, im) */
     uint32_t svoff;               /* split voxels: offset of the current voxel's plane {nx, ny, nz, pd} */

@@ -407,14 +407,16 @@ __device__ __forceinline__ void depcache_flush(const MCXKParam& g, const Shared&
 /* Voxel-exit deposits go to the LDS box when the voxel and gate fall inside it, else
    to the lane's write-combining buffer in front of the global grid.
 
-   A float32 box cell (fast build) keeps its magnitude below K_BOX_MOVE: the
-   lane whose add finds the cell above it moves K_BOX_MOVE (exactly
-   representable) from the cell to the float64 grid, as the reference moves
-   MAX_ACCUM from its float32 grid to the shadow half (src/mcx_core.cl:2882-2886).
-   Deposits therefore keep the rounding of a float32 sum below 2^11 however
-   many photons a workgroup runs, and the moved amount is exact, so nothing is
-   lost or counted twice when several lanes move at once. */
-#define K_BOX_MOVE 1024.f
+   A float32 box cell (fast build) stays within a limit around zero (MCX_BOX_LIMIT,
+   less under area sources: box_tight): what a deposit takes past an odd multiple of the limit, the
+   depositing lane moves on to the float64 grid in whole double limits, which is exact
+   (as the reference moves MAX_ACCUM from its float32 grid to the shadow half,
+   src/mcx_core.cl:2882-2886).  The adds to a cell are serial and each crossing is seen by
+   the one lane that made it: a rule by which every lane that finds the cell overfull moves
+   something takes it as far below zero as lanes deposit together (60^3 sphere, pencil
+   beam, 1e6 photons, worst cell against float64 sums: 6.4e-6 so, 7.8e-7 now).
+   A tighter limit costs moves, which contend where one voxel takes most of them: 60^3
+   sphere, pencil beam, 1e8 photons with limits 512, 256, 128, 32: 409, 409, 411, 455 ms. */
 
 /* a * b + c of factors below 2^24, at the full rate (the compiler prefers the
    quarter-rate v_mad_u64_u32) */
@@ -429,11 +431,22 @@ __device__ __forceinline__ uint32_t box_offset(const MCXKParam& g, uint32_t gate
     return mad24(mad24(mad24(gate, g.box_nz, dz), g.box_ny, dy), g.box_nx, dx);
 }
 
-/* the move of an overfull cell: idx the cell's place in the replica of the grid */
-__device__ __forceinline__ void box_move(const MCXKParam& g, const Shared& sh, BoxCell* cell, float old, uint32_t idx) {
-    const float mv = old > 0.f ? K_BOX_MOVE : -K_BOX_MOVE;
-    atomicAdd(cell, (BoxCell)(-mv));
-    grid_add(g, sh.repoff + idx, (double)mv);
+/* the move that a deposit of val brings about in a cell that held old: idx the cell's
+   place in the replica of the grid */
+__device__ __forceinline__ void box_move(const MCXKParam& g, const Shared& sh, BoxCell* cell, float old, float val,
+        uint32_t idx, float limit) {
+    const float now = old + val;    /* the cell's own sum: both round to nearest */
+
+    if (fmaxf(fabsf(old), fabsf(now)) >= limit) {
+        /* a power of two: its reciprocal and the products with it are exact */
+        const float twice = 2.f * limit, inv = 1.f / twice;
+        const float mv = (floorf(now * inv + 0.5f) - floorf(old * inv + 0.5f)) * twice;
+
+        if (mv != 0.f && fabsf(mv) < INFINITY) {
+            atomicAdd(cell, (BoxCell)(-mv));
+            grid_add(g, sh.repoff + idx, (double)mv);
+        }
+    }
 }
 
 /* binary16 bit pattern (sign bit clear) to float, exactly, subnormals included */
@@ -638,7 +651,8 @@ __device__ __forceinline__ int svmc_reflect(float n1, float4& v, Photon& s, cons
 enum {kfGscatter = 1u << 0, kfPerVoxel = 1u << 1, kfPacked = 1u << 2, kfSvmc = 1u << 3, kfRf = 1u << 4,
       kfSave = 1u << 5, kfFlux = 1u << 6, kfReflect = 1u << 7, kfPathTally = 1u << 8, kfPatterns = 1u << 9,
       kfSlots = 1u << 10, kfMoveOnly = 1u << 11, kfPhase = 1u << 12, kf2D = 1u << 13, kfPol = 1u << 14,
-      kfScatDeposit = 1u << 15, kfTraj = 1u << 16, kfCountTally = 1u << 17, kfMomTally = 1u << 18, kfRfReplay = 1u << 19, kfGates = 1u << 20
+      kfScatDeposit = 1u << 15, kfTraj = 1u << 16, kfCountTally = 1u << 17, kfMomTally = 1u << 18, kfRfReplay = 1u << 19, kfGates = 1u << 20,
+      kfTight = 1u << 21
      };
 
 __device__ __forceinline__ uint32_t features(const MCXKParam& g) {
@@ -666,6 +680,7 @@ __device__ __forceinline__ uint32_t features(const MCXKParam& g) {
          kfScatDeposit : 0u;
     w |= g.savetraj ? kfTraj : 0u;
     w |= g.maxgate > 1 ? kfGates : 0u;
+    w |= g.box_tight ? kfTight : 0u;
     w |= (replay && g.outputtype == kRF && g.omega > 0.f) ? kfRfReplay : 0u;
     return w;
 }
@@ -921,10 +936,10 @@ __device__ __forceinline__ void deposit(const MCXKParam& g, size_t repoff, uint3
 }
 
 /* the imaginary half of an RF forward deposit: into the box's second set of
-   gates when the voxel and gate fall inside it (same cell rules as
-   deposit_voxel), else straight to the grid */
+   gates when the voxel and gate fall inside it (same cell rules as the real
+   half's), else straight to the grid */
 __device__ __forceinline__ void deposit_voxel_im(const MCXKParam& g, const Shared& sh, int ox, int oy, int oz,
-        uint32_t idx1d, int tshift, float val) {
+        uint32_t idx1d, int tshift, float val, float limit) {
     const uint32_t dx = (uint32_t)(ox - (int)g.box_x0), dy = (uint32_t)(oy - (int)g.box_y0);
     const uint32_t dz = (uint32_t)(oz - (int)g.box_z0);
     const uint32_t addr = idx1d + (uint32_t)tshift * g.nvox + g.imoff;
@@ -935,10 +950,7 @@ __device__ __forceinline__ void deposit_voxel_im(const MCXKParam& g, const Share
         atomicAdd(cell, (BoxCell)val);
 #else
         const float old = atomicAdd(cell, val);
-
-        if (fabsf(old) > K_BOX_MOVE) {
-            box_move(g, sh, cell, old, addr);
-        }
+        box_move(g, sh, cell, old, val, addr, limit);
 #endif
     } else {
         deposit(g, sh.repoff, addr, val);
@@ -2296,7 +2308,7 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
         const bool moved = (cross | (FULL && hitintf)) & (oidx < g.nvox) & ((omed | isdet) != 0);
         const uint32_t flag = isdet;
         BoxCell* cell = sh.box;
-        float boxold = 0.f;
+        float boxold = 0.f, boxval = 0.f;
         uint32_t gaddr = 0, out_a = 0;
         double out_v = 0.0;
         bool evict = false;
@@ -2381,6 +2393,7 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
                 atomicAdd(cell, (BoxCell)weight);
 #else
                 boxold = atomicAdd(cell, weight);
+                boxval = weight;
 #endif
             }
 
@@ -2392,7 +2405,8 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
                reference (src/mcx_core.cl:2902-2914): its RF forward field
                stays real */
             if (FULL && (ft & kfRf) && deposits && g.srctype != kPattern && g.srctype != kPattern3D) {
-                deposit_voxel_im(g, sh, (lin0 == oidx) ? cx : -1, cy, cz, oidx, tshift, weight_im);
+                deposit_voxel_im(g, sh, (lin0 == oidx) ? cx : -1, cy, cz, oidx, tshift, weight_im,
+                                 (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
             }
         }
 
@@ -2463,10 +2477,7 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
         n1 = s.prop.w;
 #if !MCX_PARITY
 
-        if (fabsf(boxold) > K_BOX_MOVE) {
-            box_move(g, sh, cell, boxold, gaddr);
-        }
-
+        box_move(g, sh, cell, boxold, boxval, gaddr, !SIMPLE && (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
 #endif
         /* everything rare behind one test: a photon outside or in background, out of
            time, of low weight, or at a change of index */
