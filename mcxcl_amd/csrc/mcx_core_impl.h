@@ -1871,826 +1871,836 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
 
     /* once, and again after the hand-over for the lanes that run on */
     for (;;) {
-    bool put = false;
+        bool put = false;
 
-    if (alive) {
-    Photon s;
-    Moving m;
-    s.p = make_float4(0.f, 0.f, 0.f, __uint_as_float(0x7FC00000u));
-    s.v = make_float4(0.f, 0.f, 0.f, 0.f);
-    s.f = make_float4(0.f, 0.f, 0.f, 0.f);
-    s.prop = make_float4(0.f, 0.f, 0.f, 0.f);
-    s.fx = s.fy = s.fz = 0;
-    s.fw = -1;
-    s.idx1d = 0;
-    s.mediaid = __float_as_uint(g.srcparam2.w);
-    s.w0 = 0.f;
-    s.Lmove = 0.f;
-    s.esc = s.tot = 0.f;
-    s.sv = 0;
-    m.wre = m.wim = m.pathlen = m.n1 = 0.f;
-    m.isdet = m.detvox = m.launchflag = m.lin = 0;
-    m.relaunch = true;
-    m.testint = false;
+        if (alive) {
+            Photon s;
+            Moving m;
+            s.p = make_float4(0.f, 0.f, 0.f, __uint_as_float(0x7FC00000u));
+            s.v = make_float4(0.f, 0.f, 0.f, 0.f);
+            s.f = make_float4(0.f, 0.f, 0.f, 0.f);
+            s.prop = make_float4(0.f, 0.f, 0.f, 0.f);
+            s.fx = s.fy = s.fz = 0;
+            s.fw = -1;
+            s.idx1d = 0;
+            s.mediaid = __float_as_uint(g.srcparam2.w);
+            s.w0 = 0.f;
+            s.Lmove = 0.f;
+            s.esc = s.tot = 0.f;
+            s.sv = 0;
+            m.wre = m.wim = m.pathlen = m.n1 = 0.f;
+            m.isdet = m.detvox = m.launchflag = m.lin = 0;
+            m.relaunch = true;
+            m.testint = false;
 
-    if (FULL && (feat0 & kfSvmc)) {
-        s.sn = sh.pp + g.svoff;
-    }
-
-    if (moved_on) {
-        hand_copy<false>(sh, from, s, rng, idx, m);
-    } else if (g.genergy) {
-        s.esc = g.genergy[idx * 2];
-        s.tot = g.genergy[idx * 2 + 1];
-    }
-
-    /* no load is pending when the loop begins (as in getprop) */
-    pin_photon(s, rng);
-    K_PIN(idx);
-    K_PIN(m.isdet);
-    K_PIN(m.detvox);
-    K_PIN(m.launchflag);
-    K_PIN(m.lin);
-    K_PIN(m.pathlen);
-    K_PIN(m.n1);
-    K_PIN(m.wre);
-    K_PIN(m.wim);
-
-    /* the detector flag in effect: the voxel's own, except after a reflection, where
-       the reference keeps what the step found beyond the face until the photon's next
-       step inside the voxel; detvox is the voxel's own */
-    uint32_t isdet = m.isdet, detvox = m.detvox, launchflag = m.launchflag;
-    float pathlen = m.pathlen, n1 = m.n1;
-    bool relaunch = m.relaunch;
-    /* linear index of the integer position.  It is idx1d's except after a reflection,
-       when idx1d is restored while the position keeps the reflected face's index for
-       one step (at a face on the voxel's far side the next voxel's); a deposit then
-       goes by idx1d alone, past the box */
-    uint32_t lin = m.lin;
-    /* RF forward: the complex photon weight; its value at the last voxel exit is
-       read only at exits and sits in the lane scratch at rfoff (real, imaginary) */
-    struct {
-        float wre, wim;
-    } rf = {m.wre, m.wim};
-    /* split voxels: test the plane on this step (cleared once the photon crossed
-       it, set by a scattering event, a voxel change or some relaunches), and
-       whether the step ended on it (src/mcx_core.cl:2342-2343) */
-    bool testint = m.testint, hitintf = false;
-
-    for (;;) {
-        /* the wave has thinned out: its lanes move on together with the workgroup's others */
-        const uint64_t live = __ballot(true);
-        bool ended = false;   /* one exit from the loop */
-
-        if ((uint32_t)__popcll(live) <= thresh) {
-            m.wre = rf.wre;
-            m.wim = rf.wim;
-            m.pathlen = pathlen;
-            m.n1 = n1;
-            m.isdet = isdet;
-            m.detvox = detvox;
-            m.launchflag = launchflag;
-            m.lin = lin;
-            m.relaunch = relaunch;
-            m.testint = testint;
-            hand_copy<true>(sh, hand_slot(threadIdx.x >> 6,
-                                          (uint32_t)__popcll(live & ((1ull << (threadIdx.x & 63u)) - 1ull))), s, rng,
-                            idx, m);
-            put = true;
-            ended = true;
-        } else if (relaunch) {
-            if (launch_photon<SAVEDET, SIMPLE, FULL>(g, sh, s, rng, idx, launchflag, feat0)) {
-                if (g.genergy) {
-                    g.genergy[idx * 2] = s.esc;
-                    g.genergy[idx * 2 + 1] = s.tot;
-                } else {
-                    atomicAdd(sh.energy, (double)s.esc);
-                    atomicAdd(sh.energy + 1, (double)s.tot);
-                }
-
-                ended = true;
-            } else {
-                isdet = SAVEDET ? s.mediaid & K_DET_MASK : 0u;
-                s.mediaid &= K_MED_MASK;
-                n1 = s.prop.w;
-
-                if (SAVEDET) {
-                    /* a source's own label carries no detector flag: the volume's has it */
-                    detvox = SIMPLE ? detsrc : (s.idx1d < g.nvox ? media_at(g, s.idx1d) & K_DET_MASK : 0u);
-                }
-
-                if (!SIMPLE) {
-                    pin_photon(s, rng);
-                    K_PIN(isdet);
-                    K_PIN(detvox);
-                }
-
-                lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
-                relaunch = false;
-
-                if (FULL && (feat0 & kfRf)) {
-                    rf.wre = sh.pp[g.rfoff] = s.p.w;
-                    rf.wim = sh.pp[g.rfoff + 1] = 0.f;
-                }
+            if (FULL && (feat0 & kfSvmc)) {
+                s.sn = sh.pp + g.svoff;
             }
-        }
 
-        if (ended) {
-            break;
-        }
+            if (moved_on) {
+                hand_copy<false>(sh, from, s, rng, idx, m);
+            } else if (g.genergy) {
+                s.esc = g.genergy[idx * 2];
+                s.tot = g.genergy[idx * 2 + 1];
+            }
 
-        float4& p = s.p;
-        float4& v = s.v;
-        float4& f = s.f;
-        /* one scalar register holds what the run uses; hidden from the compiler at each
-           step, or every test would be hoisted into a register pair of its own */
-        uint32_t ft = feat0;
-        asm("" : "+s"(ft));
+            /* no load is pending when the loop begins (as in getprop) */
+            pin_photon(s, rng);
+            K_PIN(idx);
+            K_PIN(m.isdet);
+            K_PIN(m.detvox);
+            K_PIN(m.launchflag);
+            K_PIN(m.lin);
+            K_PIN(m.pathlen);
+            K_PIN(m.n1);
+            K_PIN(m.wre);
+            K_PIN(m.wim);
 
-        if (f.x <= 0.f) {
-            f.x = rng.scatlen();
+            /* the detector flag in effect: the voxel's own, except after a reflection, where
+               the reference keeps what the step found beyond the face until the photon's next
+               step inside the voxel; detvox is the voxel's own */
+            uint32_t isdet = m.isdet, detvox = m.detvox, launchflag = m.launchflag;
+            float pathlen = m.pathlen, n1 = m.n1;
+            bool relaunch = m.relaunch;
+            /* linear index of the integer position.  It is idx1d's except after a reflection,
+               when idx1d is restored while the position keeps the reflected face's index for
+               one step (at a face on the voxel's far side the next voxel's); a deposit then
+               goes by idx1d alone, past the box */
+            uint32_t lin = m.lin;
+            /* RF forward: the complex photon weight; its value at the last voxel exit is
+               read only at exits and sits in the lane scratch at rfoff (real, imaginary) */
+            struct {
+                float wre, wim;
+            } rf = {m.wre, m.wim};
+            /* split voxels: test the plane on this step (cleared once the photon crossed
+               it, set by a scattering event, a voxel change or some relaunches), and
+               whether the step ended on it (src/mcx_core.cl:2342-2343) */
+            bool testint = m.testint, hitintf = false;
 
-            if (v.w != K_EPS) {
-                float cphi = 1.f, sphi = 0.f, theta = 0.f, stheta, ctheta, tmp0 = 0.f;
+            for (;;) {
+                /* the wave has thinned out: its lanes move on together with the workgroup's others */
+                const uint64_t live = __ballot(true);
+                bool ended = false;   /* one exit from the loop */
 
-                if (FULL && (ft & kfPol) && !(ft & kf2D)) {
-                    /* polarised media (src/mcx_core.cl:2454-2468): (theta, phi) by rejection
-                       against I(theta, phi) = S11 I + S12 (Q cos 2phi + U sin 2phi) of the
-                       medium's table, the forward entry as the bound */
-                    const uint32_t lab = s.mediaid & K_MED_MASK;
-                    const uint32_t ipol = K_NANGLES * (lab ? lab - 1 : 0u);   /* scattering needs mus > 0: label >= 1 */
-                    const float4 st = stokes_get(g, sh.pp);
-                    float ii, sin2phi, cos2phi;
-#if MCX_PARITY
-                    float i0;
-
-                    do {
-                        theta = kacos(2.f * rng.next() - 1.f);
-                        tmp0 = K_TWO_PI * rng.next();
-                        ksincos(2.f * tmp0, &sin2phi, &cos2phi);
-                        const float4 m0 = g.smatrix[ipol];
-                        i0 = m0.x * st.x + m0.y * (st.y * cos2phi + st.z * sin2phi);
-                        const float4 mt = g.smatrix[ipol + (uint32_t)(theta * (float)K_NANGLES * (K_R_PI - K_EPS))];
-                        ii = mt.x * st.x + mt.y * (st.y * cos2phi + st.z * sin2phi);
-                    } while (rng.next() * i0 >= ii);
-
-                    ksincos(theta, &stheta, &ctheta);
-#else
-                    /* the same distribution in fewer draws: theta from its marginal, S11 of
-                       its table bin times sin(theta) (a CDF over the bins, uniform in
-                       cos(theta) inside one), then phi given theta by rejection against
-                       S11 I + |S12| |(Q, U)|, which accepts at least half the draws (the
-                       joint rejection above takes ~17 rounds for 0.3 um spheres) */
-                    const float* cdf = g.polcdf + (K_NANGLES + 1) * (1u + (lab ? lab - 1 : 0u));
-                    const float u = rng.next();
-                    uint32_t lo = 0, hi = K_NANGLES;
-
-                    while (hi - lo > 1) {
-                        const uint32_t mid = (lo + hi) >> 1;
-
-                        if (cdf[mid] <= u) {
-                            lo = mid;
+                if ((uint32_t)__popcll(live) <= thresh) {
+                    m.wre = rf.wre;
+                    m.wim = rf.wim;
+                    m.pathlen = pathlen;
+                    m.n1 = n1;
+                    m.isdet = isdet;
+                    m.detvox = detvox;
+                    m.launchflag = launchflag;
+                    m.lin = lin;
+                    m.relaunch = relaunch;
+                    m.testint = testint;
+                    const uint64_t below = (1ull << (threadIdx.x & 63u)) - 1ull;
+                    hand_copy<true>(sh, hand_slot(threadIdx.x >> 6, (uint32_t)__popcll(live & below)), s, rng, idx, m);
+                    put = true;
+                    ended = true;
+                } else if (relaunch) {
+                    if (launch_photon<SAVEDET, SIMPLE, FULL>(g, sh, s, rng, idx, launchflag, feat0)) {
+                        if (g.genergy) {
+                            g.genergy[idx * 2] = s.esc;
+                            g.genergy[idx * 2 + 1] = s.tot;
                         } else {
-                            hi = mid;
+                            atomicAdd(sh.energy, (double)s.esc);
+                            atomicAdd(sh.energy + 1, (double)s.tot);
+                        }
+
+                        ended = true;
+                    } else {
+                        isdet = SAVEDET ? s.mediaid & K_DET_MASK : 0u;
+                        s.mediaid &= K_MED_MASK;
+                        n1 = s.prop.w;
+
+                        if (SAVEDET) {
+                            /* a source's own label carries no detector flag: the volume's has it */
+                            detvox = SIMPLE ? detsrc : (s.idx1d < g.nvox ? media_at(g, s.idx1d) & K_DET_MASK : 0u);
+                        }
+
+                        if (!SIMPLE) {
+                            pin_photon(s, rng);
+                            K_PIN(isdet);
+                            K_PIN(detvox);
+                        }
+
+                        lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+                        relaunch = false;
+
+                        if (FULL && (feat0 & kfRf)) {
+                            rf.wre = sh.pp[g.rfoff] = s.p.w;
+                            rf.wim = sh.pp[g.rfoff + 1] = 0.f;
                         }
                     }
-
-                    const float ce0 = g.polcdf[lo], ce1 = g.polcdf[lo + 1];
-                    ctheta = ce1 + (ce0 - ce1) * rng.next();
-                    theta = kacos(ctheta);
-                    stheta = ksin_acos(ctheta);
-                    const float4 mt = g.smatrix[ipol + lo];
-                    const float bound = mt.x * st.x +
-                                        fabsf(mt.y) * ksqrt(st.y * st.y + st.z * st.z);
-
-                    do {
-                        tmp0 = K_TWO_PI * rng.next();
-                        ksincos(2.f * tmp0, &sin2phi, &cos2phi);
-                        ii = mt.x * st.x + mt.y * (st.y * cos2phi + st.z * sin2phi);
-                    } while (rng.next() * bound >= ii);
-#endif
-                    ksincos(tmp0, &sphi, &cphi);
-                } else {
-                if (SIMPLE || !(ft & kf2D)) {
-                    const float turn = rng.next();
-                    tmp0 = K_TWO_PI * turn;
-                    ksincos_turn(turn, &sphi, &cphi);
                 }
 
-                if (!SIMPLE && (ft & kfPhase)) {
-                    tmp0 = rng.next() * (float)(g.nphase - 1);
-                    theta = tmp0 - (float)((int)tmp0);
-                    uint32_t i0 = (uint32_t)tmp0 >= g.nphase ? g.nphase - 1 : (uint32_t)(int)tmp0;
-                    uint32_t i1 = (uint32_t)tmp0 + 1 >= g.nphase ? g.nphase - 1 : (uint32_t)((int)tmp0 + 1);
-                    tmp0 = (1.f - theta) * sh.invcdf[i0] + theta * sh.invcdf[i1];
-                    stheta = ksin_acos(tmp0);
-                    ctheta = tmp0;
+                if (ended) {
+                    break;
+                }
 
-                    if (FULL && (ft & kfPol)) {
-                        theta = kacos(tmp0);    /* the angle the Stokes update takes (2D polarised runs) */
-                    }
-                } else {
-                    tmp0 = ((ft & kfGscatter) && v.w > (float)g.gscatter) ? 0.f : s.prop.z;
+                float4& p = s.p;
+                float4& v = s.v;
+                float4& f = s.f;
+                /* one scalar register holds what the run uses; hidden from the compiler at each
+                   step, or every test would be hoisted into a register pair of its own */
+                uint32_t ft = feat0;
+                asm("" : "+s"(ft));
 
-                    if (fabsf(tmp0) > K_EPS) {
-                        tmp0 = kdiv(1.f - s.prop.z * s.prop.z, 1.f - s.prop.z + 2.f * s.prop.z * rng.next());
-                        tmp0 *= tmp0;
-                        tmp0 = kdiv(1.f + s.prop.z * s.prop.z - tmp0, 2.f * s.prop.z);
-                        tmp0 = fmaxf(-1.f, fminf(1.f, tmp0));
-                        stheta = ksin_acos(tmp0);
-                        ctheta = tmp0;
+                if (f.x <= 0.f) {
+                    f.x = rng.scatlen();
 
-                        if (FULL && (ft & kfPol)) {
-                            theta = kacos(tmp0);
-                        }
-                    } else {
+                    if (v.w != K_EPS) {
+                        float cphi = 1.f, sphi = 0.f, theta = 0.f, stheta, ctheta, tmp0 = 0.f;
+
+                        if (FULL && (ft & kfPol) && !(ft & kf2D)) {
+                            /* polarised media (src/mcx_core.cl:2454-2468): (theta, phi) by rejection
+                               against I(theta, phi) = S11 I + S12 (Q cos 2phi + U sin 2phi) of the
+                               medium's table, the forward entry as the bound */
+                            const uint32_t lab = s.mediaid & K_MED_MASK;
+                            /* scattering needs mus > 0: label >= 1 */
+                            const uint32_t ipol = K_NANGLES * (lab ? lab - 1 : 0u);
+                            const float4 st = stokes_get(g, sh.pp);
+                            float ii, sin2phi, cos2phi;
 #if MCX_PARITY
-                        theta = kacos(2.f * rng.next() - 1.f);
-                        ksincos(theta, &stheta, &ctheta);
+                            float i0;
+
+                            do {
+                                theta = kacos(2.f * rng.next() - 1.f);
+                                tmp0 = K_TWO_PI * rng.next();
+                                ksincos(2.f * tmp0, &sin2phi, &cos2phi);
+                                const float4 m0 = g.smatrix[ipol];
+                                i0 = m0.x * st.x + m0.y * (st.y * cos2phi + st.z * sin2phi);
+                                const float4 mt = g.smatrix[ipol + (uint32_t)(theta * (float)K_NANGLES *
+                                                                             (K_R_PI - K_EPS))];
+                                ii = mt.x * st.x + mt.y * (st.y * cos2phi + st.z * sin2phi);
+                            } while (rng.next() * i0 >= ii);
+
+                            ksincos(theta, &stheta, &ctheta);
 #else
-                        ctheta = 2.f * rng.next() - 1.f;
-                        stheta = ksin_acos(ctheta);
+                            /* the same distribution in fewer draws: theta from its marginal, S11 of
+                               its table bin times sin(theta) (a CDF over the bins, uniform in
+                               cos(theta) inside one), then phi given theta by rejection against
+                               S11 I + |S12| |(Q, U)|, which accepts at least half the draws (the
+                               joint rejection above takes ~17 rounds for 0.3 um spheres) */
+                            const float* cdf = g.polcdf + (K_NANGLES + 1) * (1u + (lab ? lab - 1 : 0u));
+                            const float u = rng.next();
+                            uint32_t lo = 0, hi = K_NANGLES;
+
+                            while (hi - lo > 1) {
+                                const uint32_t mid = (lo + hi) >> 1;
+
+                                if (cdf[mid] <= u) {
+                                    lo = mid;
+                                } else {
+                                    hi = mid;
+                                }
+                            }
+
+                            const float ce0 = g.polcdf[lo], ce1 = g.polcdf[lo + 1];
+                            ctheta = ce1 + (ce0 - ce1) * rng.next();
+                            theta = kacos(ctheta);
+                            stheta = ksin_acos(ctheta);
+                            const float4 mt = g.smatrix[ipol + lo];
+                            const float bound = mt.x * st.x +
+                                                fabsf(mt.y) * ksqrt(st.y * st.y + st.z * st.z);
+
+                            do {
+                                tmp0 = K_TWO_PI * rng.next();
+                                ksincos(2.f * tmp0, &sin2phi, &cos2phi);
+                                ii = mt.x * st.x + mt.y * (st.y * cos2phi + st.z * sin2phi);
+                            } while (rng.next() * bound >= ii);
+#endif
+                            ksincos(tmp0, &sphi, &cphi);
+                        } else {
+                            if (SIMPLE || !(ft & kf2D)) {
+                                const float turn = rng.next();
+                                tmp0 = K_TWO_PI * turn;
+                                ksincos_turn(turn, &sphi, &cphi);
+                            }
+
+                            if (!SIMPLE && (ft & kfPhase)) {
+                                tmp0 = rng.next() * (float)(g.nphase - 1);
+                                theta = tmp0 - (float)((int)tmp0);
+                                uint32_t i0 = (uint32_t)tmp0 >= g.nphase ? g.nphase - 1 : (uint32_t)(int)tmp0;
+                                uint32_t i1 = (uint32_t)tmp0 + 1 >= g.nphase ? g.nphase - 1 : (uint32_t)((int)tmp0 + 1);
+                                tmp0 = (1.f - theta) * sh.invcdf[i0] + theta * sh.invcdf[i1];
+                                stheta = ksin_acos(tmp0);
+                                ctheta = tmp0;
+
+                                if (FULL && (ft & kfPol)) {
+                                    theta = kacos(tmp0);    /* the angle the Stokes update takes (2D polarised runs) */
+                                }
+                            } else {
+                                tmp0 = ((ft & kfGscatter) && v.w > (float)g.gscatter) ? 0.f : s.prop.z;
+
+                                if (fabsf(tmp0) > K_EPS) {
+                                    tmp0 = kdiv(1.f - s.prop.z * s.prop.z,
+                                                1.f - s.prop.z + 2.f * s.prop.z * rng.next());
+                                    tmp0 *= tmp0;
+                                    tmp0 = kdiv(1.f + s.prop.z * s.prop.z - tmp0, 2.f * s.prop.z);
+                                    tmp0 = fmaxf(-1.f, fminf(1.f, tmp0));
+                                    stheta = ksin_acos(tmp0);
+                                    ctheta = tmp0;
+
+                                    if (FULL && (ft & kfPol)) {
+                                        theta = kacos(tmp0);
+                                    }
+                                } else {
+#if MCX_PARITY
+                                    theta = kacos(2.f * rng.next() - 1.f);
+                                    ksincos(theta, &stheta, &ctheta);
+#else
+                                    ctheta = 2.f * rng.next() - 1.f;
+                                    stheta = ksin_acos(ctheta);
+
+                                    if (FULL && (ft & kfPol)) {
+                                        theta = kacos(ctheta);
+                                    }
+#endif
+                                }
+                            }
+                        }
+
+                        /* per-medium tallies: a split voxel's current side (src/mcx_core.cl:2502-2540) */
+                        const uint32_t tlab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : s.mediaid;
+
+                        if (SAVEDET && tlab > 0) {
+                            if (ft & kfCountTally) {
+                                uint32_t* cnt = (uint32_t*)sh.pp;
+                                cnt[tlab - 1]++;
+                            }
+
+                            if (ft & kfMomTally) {
+                                sh.pp[g.maxmedia * (((g.savedetflag >> 1) & 1) + ((g.savedetflag >> 2) & 1)) + tlab -
+                                      1] +=
+                                    1.f - ctheta;
+                            }
+                        }
+
+                        const float4 olddir = v;
+
+                        if (!SIMPLE && (ft & kf2D)) {
+                            rotatevector2d(v, (rng.next() > 0.5f ? stheta : -stheta), ctheta, (int)g.is2d);
+                        } else {
+                            rotatevector(v, stheta, ctheta, sphi, cphi);
+                        }
+
+                        v.w += 1.f;
 
                         if (FULL && (ft & kfPol)) {
-                            theta = kacos(ctheta);
+                            /* :2550-2565; in 2D the reference samples by HG with the medium's g and
+                               passes the sampled cosine (tmp0) where the azimuth goes */
+                            float4 st = stokes_get(g, sh.pp);
+                            update_stokes(g, st, theta, tmp0, olddir, v, s.mediaid);
+                            stokes_put(g, sh.pp, st);
                         }
-#endif
+
+                        if (!SIMPLE && (ft & kfScatDeposit) && (FULL || g.outputtype == kWP || g.outputtype == kDCS)) {
+                            /* replay deposits at each scattering site (src/mcx_core.cl:2568-2623):
+                               w (WP), (1 - cos theta) w (DCS), tof w (WPTOF), w e^{i omega tof} (RFmus) */
+                            uint32_t pid = photon_index(g, idx, f.w) - 1;
+                            float im = 0.f;
+                            tmp0 = (g.outputtype == kDCS) ? (1.f - ctheta) : 1.f;
+
+                            if (FULL && g.outputtype == kRFmus) {
+                                const float rw = g.replayweight[pid];
+                                tmp0 = rw * sh.pp[g.w0offset + g.srcnum];
+                                im = rw * sh.pp[g.w0offset + g.srcnum + 1];
+                            } else if (FULL && g.outputtype == kWPTOF) {
+                                tmp0 = g.replaytof[pid];
+                                tmp0 *= g.replayweight[pid];
+                            } else {
+                                tmp0 *= g.replayweight[pid];
+                            }
+
+                            int tshift = gate_of(g, g.replaytof[pid]) +
+                                         ((g.replaydet == -1) ?
+                                          (((g.replaydetid[pid] & 0xFFFF) - 1) * (int)g.maxgate) : 0);
+
+                            if (g.extrasrclen && g.srcid < 0) {
+                                tshift += ((int)sh.pp[g.w0offset - 1] - 1) * ((g.replaydet == -1) ? (int)g.detnum : 1) *
+                                          (int)g.maxgate;
+                            }
+
+                            deposit(g, sh.repoff, s.idx1d + (uint32_t)tshift * g.nvox, tmp0);
+
+                            if (FULL && g.outputtype == kRFmus) {
+                                deposit(g, sh.repoff, s.idx1d + (uint32_t)tshift * g.nvox + g.imoff, im);
+                            }
+                        }
+
+                        if (FULL && (ft & kfTraj)) {
+                            save_traj(g, p, traj_index(g, idx, f.w), sh.pp[g.w0offset - 1], sh.pp + g.stokesoff);
+                        }
+                    }
+
+                    v.w = (float)(int)v.w;
+
+                    if (FULL && (ft & kfSvmc)) {
+                        testint = true;
                     }
                 }
+
+                /* s.prop holds the properties of the photon's voxel and n1 its index; split
+                   voxels: the side is taken again from the position at every step
+                   (src/mcx_core.cl:2656-2672) */
+                if (FULL && (ft & kfSvmc)) {
+                    n1 = s.prop.w;
+                    s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
                 }
 
-                /* per-medium tallies: a split voxel's current side (src/mcx_core.cl:2502-2540) */
-                const uint32_t tlab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : s.mediaid;
+                int face;
+                f.z = hitgrid(p, v, s.fx, s.fy, s.fz, &face);
+                float gfac = 1.f;
 
-                if (SAVEDET && tlab > 0) {
-                    if (ft & kfCountTally) {
-                        uint32_t* cnt = (uint32_t*)sh.pp;
-                        cnt[tlab - 1]++;
-                    }
+                if (ft & kfGscatter) {
+                    gfac = (v.w + 1.f > (float)g.gscatter ? (1.f - s.prop.z) : 1.f);
+                    K_PIN(gfac);
+                }
 
-                    if (ft & kfMomTally) {
-                        sh.pp[g.maxmedia * (((g.savedetflag >> 1) & 1) + ((g.savedetflag >> 2) & 1)) + tlab - 1] +=
-                            1.f - ctheta;
+                if (SIMPLE) {
+                    /* one grid atomic in flight per lane: where the atomics bound the run, more of
+                       them queue in the memory system without being served any faster (60^3
+                       sphere, 1e8 photons: 432 ms unbounded, 418 ms); elsewhere no cost */
+                    asm("s_waitcnt vmcnt(0)" : "+v"(s.prop.y));
+                }
+
+                float slen = f.z * s.prop.y * gfac;
+                /* the scattering site comes before the face */
+                bool stay = !(slen < f.x);
+                slen = stay ? f.x : slen;
+                f.z = kdiv(slen, s.prop.y * gfac);
+
+                if (FULL && (ft & kfSvmc)) {
+                    /* the step ends on the voxel's plane when it crosses it (src/mcx_core.cl:2684-2701) */
+                    hitintf = false;
+
+                    if (K_SV_ISSPLIT(s.sv) && testint) {
+                        float len = f.z;
+                        hitintf = svmc_ray_plane(s, v, gfac, &len, &slen);
+                        f.z = len;
                     }
                 }
 
-                const float4 olddir = v;
+                pathlen += f.z;
+                p.x = p.x + f.z * v.x;
+                p.y = p.y + f.z * v.y;
+                p.z = p.z + f.z * v.z;
+                K_PIN(p.x);
+                K_PIN(p.y);
+                K_PIN(p.z);
 
-                if (!SIMPLE && (ft & kf2D)) {
-                    rotatevector2d(v, (rng.next() > 0.5f ? stheta : -stheta), ctheta, (int)g.is2d);
+                stay = stay | (FULL && hitintf);
+                float vface = v.z;
+                int lstep = (int)g.dimxy;
+                vface = (face == 1) ? v.y : vface;
+                lstep = (face == 1) ? (int)g.dimx : lstep;
+                vface = (face == 0) ? v.x : vface;
+                lstep = (face == 0) ? 1 : lstep;
+                const int sgn = stay ? 0 : (vface > 0.f ? 1 : -1);
+                const uint32_t lin0 = lin;
+                lin += (uint32_t)(stay ? 0 : (vface > 0.f ? lstep : -lstep));
+                /* the voxel the photon leaves, and the one it is in now */
+                const int cx = s.fx, cy = s.fy, cz = s.fz;
+                s.fx += (face == 0) ? sgn : 0;
+                s.fy += (face == 1) ? sgn : 0;
+                s.fz += (face == 2) ? sgn : 0;
+                K_PIN(s.fx);
+                K_PIN(s.fy);
+                K_PIN(s.fz);
+
+                /* the label is loaded only where the voxel changes, ahead of the arithmetic
+                   that does not need it */
+                const bool in = inside(g, s.fx, s.fy, s.fz);
+                const uint32_t oidx = s.idx1d, omed = s.mediaid;
+                s.idx1d = in ? lin : (((s.fx | s.fy | s.fz) < 0) ? K_OUT_MIN : K_OUT_MAX);
+                const bool cross = s.idx1d != oidx;
+                uint32_t lab = 0;
+
+                if (in & cross) {
+                    lab = ((const K_GLOBAL uint32_t*)mediabase)[s.idx1d];
+                }
+
+                if (FULL && (ft & kfRf)) {
+                    /* RF forward (src/mcx_core.cl:2750-2760): w <- w exp(-(mua + i omega n / c0) ds),
+                       p.w its magnitude */
+                    const float att = kexp(-s.prop.x * f.z);
+                    float rs, rc;
+                    ksincos(g.omega * s.prop.w * g.oneoverc0 * f.z, &rs, &rc);
+                    const float tre = att * (rf.wre * rc + rf.wim * rs);
+                    const float tim = att * (-rf.wre * rs + rf.wim * rc);
+                    rf.wre = tre;
+                    rf.wim = tim;
+                    p.w = ksqrt(rf.wre * rf.wre + rf.wim * rf.wim);
                 } else {
-                    rotatevector(v, stheta, ctheta, sphi, cphi);
+                    p.w *= kexp(-s.prop.x * f.z);
                 }
 
-                v.w += 1.f;
+                f.x -= slen;
+                f.y += f.z * s.prop.w * hold.oneoverc0;
 
-                if (FULL && (ft & kfPol)) {
-                    /* :2550-2565; in 2D the reference samples by HG with the medium's g and
-                       passes the sampled cosine (tmp0) where the azimuth goes */
-                    float4 st = stokes_get(g, sh.pp);
-                    update_stokes(g, st, theta, tmp0, olddir, v, s.mediaid);
-                    stokes_put(g, sh.pp, st);
-                }
+                if (SAVEDET && (ft & kfPathTally)) {
+                    const uint32_t plab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : s.mediaid;
 
-                if (!SIMPLE && (ft & kfScatDeposit) && (FULL || g.outputtype == kWP || g.outputtype == kDCS)) {
-                    /* replay deposits at each scattering site (src/mcx_core.cl:2568-2623):
-                       w (WP), (1 - cos theta) w (DCS), tof w (WPTOF), w e^{i omega tof} (RFmus) */
-                    uint32_t pid = photon_index(g, idx, f.w) - 1;
-                    float im = 0.f;
-                    tmp0 = (g.outputtype == kDCS) ? (1.f - ctheta) : 1.f;
-
-                    if (FULL && g.outputtype == kRFmus) {
-                        const float rw = g.replayweight[pid];
-                        tmp0 = rw * sh.pp[g.w0offset + g.srcnum];
-                        im = rw * sh.pp[g.w0offset + g.srcnum + 1];
-                    } else if (FULL && g.outputtype == kWPTOF) {
-                        tmp0 = g.replaytof[pid];
-                        tmp0 *= g.replayweight[pid];
-                    } else {
-                        tmp0 *= g.replayweight[pid];
+                    if (plab > 0) {
+                        atomicAdd(&sh.pp[g.maxmedia * ((ft & kfCountTally) ? 1u : 0u) + plab - 1], f.z);
                     }
+                }
 
-                    int tshift = gate_of(g, g.replaytof[pid]) +
+                /* a photon that left its voxel deposits there; one crossing out of a background
+                   voxel keeps label 0 (src/mcx_core.cl:2806-2930) */
+                const bool moved = (cross | (FULL && hitintf)) & (oidx < g.nvox) & ((omed | isdet) != 0);
+                const uint32_t flag = isdet;
+                BoxCell* cell = sh.box;
+                float boxold = 0.f, boxval = 0.f;
+                uint32_t gaddr = 0, out_a = 0;
+                double out_v = 0.0;
+                bool evict = false;
+
+                /* the deposit: computed for every lane, most of a wave's lanes deposit in most
+                   steps */
+                float weight = 0.f, weight_im = 0.f;
+                int tshift = 0;
+
+                if (ft & kfGates) {
+                    tshift = (int)floorf((f.y - g.twin0) * hold.Rtstep);
+                    tshift = tshift > (int)g.maxgate - 1 ? (int)g.maxgate - 1 : tshift;
+                }
+
+                bool deposits = moved & ((ft & kfSave) != 0) & (f.y >= g.twin0) & (f.y < g.twin1);
+
+                if (FULL && (ft & kfRf)) {
+                    /* RF forward (src/mcx_core.cl:2833-2839): (w0 - w) / (mua + i omega n / c0) */
+                    const float w0re = sh.pp[g.rfoff], w0im = sh.pp[g.rfoff + 1];
+                    const float dre = w0re - rf.wre, dim = w0im - rf.wim;
+                    const float aim = g.omega * s.prop.w * g.oneoverc0;
+                    const float amag2 = s.prop.x * s.prop.x + aim * aim;
+                    weight = (amag2 < K_EPS) ? (w0re * pathlen) : kdiv(dre * s.prop.x + dim * aim, amag2);
+                    weight_im = (amag2 < K_EPS) ? (w0im * pathlen) : kdiv(dim * s.prop.x - dre * aim, amag2);
+                } else if (ft & kfFlux) {
+                    float q = kdiv(s.w0 - p.w, s.prop.x);
+                    K_PIN(q);
+                    weight = (s.prop.x < K_EPS) ? (s.w0 * pathlen) : q;
+                } else if (g.outputtype == kEnergy) {
+                    weight = s.w0 - p.w;
+                } else if (!SIMPLE && g.seed == K_SEED_FROM_FILE) {
+                    if (deposits && (g.outputtype == kJacobian ||
+                                     (FULL && (g.outputtype == kRF || g.outputtype == kWLTOF)))) {
+                        /* replay path deposits (src/mcx_core.cl:2845-2858): w L (J),
+                           -w L e^{i omega tof} (RF), tof w L (WLTOF) */
+                        uint32_t pid = photon_index(g, idx, f.w) - 1;
+                        weight = g.replayweight[pid] * pathlen;
+                        tshift = gate_of(g, g.replaytof[pid]) +
                                  ((g.replaydet == -1) ? (((g.replaydetid[pid] & 0xFFFF) - 1) * (int)g.maxgate) : 0);
 
-                    if (g.extrasrclen && g.srcid < 0) {
-                        tshift += ((int)sh.pp[g.w0offset - 1] - 1) * ((g.replaydet == -1) ? (int)g.detnum : 1) *
-                                  (int)g.maxgate;
+                        if (FULL && g.outputtype == kRF) {
+                            weight_im = -weight * sh.pp[g.w0offset + g.srcnum + 1];
+                            weight = -weight * sh.pp[g.w0offset + g.srcnum];
+                        } else if (FULL && g.outputtype == kWLTOF) {
+                            weight = weight * g.replaytof[pid];
+                        }
                     }
+                } else if (g.outputtype == kL) {
+                    weight = s.w0 * pathlen;
+                }
 
-                    deposit(g, sh.repoff, s.idx1d + (uint32_t)tshift * g.nvox, tmp0);
+                if (!SIMPLE && (ft & kfSlots)) {
+                    tshift += ((int)sh.pp[g.w0offset - 1] - 1) * ((g.replaydet == -1) ? (int)g.detnum : 1) *
+                              (int)g.maxgate;
+                }
 
-                    if (FULL && g.outputtype == kRFmus) {
-                        deposit(g, sh.repoff, s.idx1d + (uint32_t)tshift * g.nvox + g.imoff, im);
+                deposits = deposits & (fabsf(weight) > 0.f);
+
+                if (FULL && (ft & kfPatterns)) {
+                    if (deposits) {
+                        /* several patterns share the photon: one interleaved slot per pattern
+                           (src/mcx_core.cl:2902-2914), straight to the grid */
+                        const uint32_t base = (oidx + (uint32_t)tshift * g.nvox) * g.npattern;
+
+                        for (uint32_t i = 0; i < g.npattern; i++) {
+                            const float pw = sh.pp[g.w0offset + i];
+
+                            if (fabsf(pw) > 0.f) {
+                                deposit(g, sh.repoff, base + i, weight * pw);
+                            }
+                        }
                     }
-                }
+                } else {
+                    const uint32_t dx = (uint32_t)(cx - (int)g.box_x0), dy = (uint32_t)(cy - (int)g.box_y0);
+                    const uint32_t dz = (uint32_t)(cz - (int)g.box_z0);
+                    const bool inbox = (dx < g.box_nx) & (dy < g.box_ny) & (dz < g.box_nz) &
+                                       ((uint32_t)tshift < g.box_ng) & (lin0 == oidx);
+                    gaddr = oidx + (uint32_t)tshift * g.nvox;
 
-                if (FULL && (ft & kfTraj)) {
-                    save_traj(g, p, traj_index(g, idx, f.w), sh.pp[g.w0offset - 1], sh.pp + g.stokesoff);
-                }
-            }
-
-            v.w = (float)(int)v.w;
-
-            if (FULL && (ft & kfSvmc)) {
-                testint = true;
-            }
-        }
-
-        /* s.prop holds the properties of the photon's voxel and n1 its index; split
-           voxels: the side is taken again from the position at every step
-           (src/mcx_core.cl:2656-2672) */
-        if (FULL && (ft & kfSvmc)) {
-            n1 = s.prop.w;
-            s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
-        }
-
-        int face;
-        f.z = hitgrid(p, v, s.fx, s.fy, s.fz, &face);
-        float gfac = 1.f;
-
-        if (ft & kfGscatter) {
-            gfac = (v.w + 1.f > (float)g.gscatter ? (1.f - s.prop.z) : 1.f);
-            K_PIN(gfac);
-        }
-
-        if (SIMPLE) {
-            /* one grid atomic in flight per lane: where the atomics bound the run, more of
-               them queue in the memory system without being served any faster (60^3
-               sphere, 1e8 photons: 432 ms unbounded, 418 ms); elsewhere no cost */
-            asm("s_waitcnt vmcnt(0)" : "+v"(s.prop.y));
-        }
-
-        float slen = f.z * s.prop.y * gfac;
-        /* the scattering site comes before the face */
-        bool stay = !(slen < f.x);
-        slen = stay ? f.x : slen;
-        f.z = kdiv(slen, s.prop.y * gfac);
-
-        if (FULL && (ft & kfSvmc)) {
-            /* the step ends on the voxel's plane when it crosses it (src/mcx_core.cl:2684-2701) */
-            hitintf = false;
-
-            if (K_SV_ISSPLIT(s.sv) && testint) {
-                float len = f.z;
-                hitintf = svmc_ray_plane(s, v, gfac, &len, &slen);
-                f.z = len;
-            }
-        }
-
-        pathlen += f.z;
-        p.x = p.x + f.z * v.x;
-        p.y = p.y + f.z * v.y;
-        p.z = p.z + f.z * v.z;
-        K_PIN(p.x);
-        K_PIN(p.y);
-        K_PIN(p.z);
-
-        stay = stay | (FULL && hitintf);
-        float vface = v.z;
-        int lstep = (int)g.dimxy;
-        vface = (face == 1) ? v.y : vface;
-        lstep = (face == 1) ? (int)g.dimx : lstep;
-        vface = (face == 0) ? v.x : vface;
-        lstep = (face == 0) ? 1 : lstep;
-        const int sgn = stay ? 0 : (vface > 0.f ? 1 : -1);
-        const uint32_t lin0 = lin;
-        lin += (uint32_t)(stay ? 0 : (vface > 0.f ? lstep : -lstep));
-        /* the voxel the photon leaves, and the one it is in now */
-        const int cx = s.fx, cy = s.fy, cz = s.fz;
-        s.fx += (face == 0) ? sgn : 0;
-        s.fy += (face == 1) ? sgn : 0;
-        s.fz += (face == 2) ? sgn : 0;
-        K_PIN(s.fx);
-        K_PIN(s.fy);
-        K_PIN(s.fz);
-
-        /* the label is loaded only where the voxel changes, ahead of the arithmetic
-           that does not need it */
-        const bool in = inside(g, s.fx, s.fy, s.fz);
-        const uint32_t oidx = s.idx1d, omed = s.mediaid;
-        s.idx1d = in ? lin : (((s.fx | s.fy | s.fz) < 0) ? K_OUT_MIN : K_OUT_MAX);
-        const bool cross = s.idx1d != oidx;
-        uint32_t lab = 0;
-
-        if (in & cross) {
-            lab = ((const K_GLOBAL uint32_t*)mediabase)[s.idx1d];
-        }
-
-        if (FULL && (ft & kfRf)) {
-            /* RF forward (src/mcx_core.cl:2750-2760): w <- w exp(-(mua + i omega n / c0) ds),
-               p.w its magnitude */
-            const float att = kexp(-s.prop.x * f.z);
-            float rs, rc;
-            ksincos(g.omega * s.prop.w * g.oneoverc0 * f.z, &rs, &rc);
-            const float tre = att * (rf.wre * rc + rf.wim * rs);
-            const float tim = att * (-rf.wre * rs + rf.wim * rc);
-            rf.wre = tre;
-            rf.wim = tim;
-            p.w = ksqrt(rf.wre * rf.wre + rf.wim * rf.wim);
-        } else {
-            p.w *= kexp(-s.prop.x * f.z);
-        }
-
-        f.x -= slen;
-        f.y += f.z * s.prop.w * hold.oneoverc0;
-
-        if (SAVEDET && (ft & kfPathTally)) {
-            const uint32_t plab = (FULL && (ft & kfSvmc)) ? K_SV_CURLABEL(s.sv) : s.mediaid;
-
-            if (plab > 0) {
-                atomicAdd(&sh.pp[g.maxmedia * ((ft & kfCountTally) ? 1u : 0u) + plab - 1], f.z);
-            }
-        }
-
-        /* a photon that left its voxel deposits there; one crossing out of a background
-           voxel keeps label 0 (src/mcx_core.cl:2806-2930) */
-        const bool moved = (cross | (FULL && hitintf)) & (oidx < g.nvox) & ((omed | isdet) != 0);
-        const uint32_t flag = isdet;
-        BoxCell* cell = sh.box;
-        float boxold = 0.f, boxval = 0.f;
-        uint32_t gaddr = 0, out_a = 0;
-        double out_v = 0.0;
-        bool evict = false;
-
-        /* the deposit: computed for every lane, most of a wave's lanes deposit in most
-           steps */
-        float weight = 0.f, weight_im = 0.f;
-        int tshift = 0;
-
-        if (ft & kfGates) {
-            tshift = (int)floorf((f.y - g.twin0) * hold.Rtstep);
-            tshift = tshift > (int)g.maxgate - 1 ? (int)g.maxgate - 1 : tshift;
-        }
-
-        bool deposits = moved & ((ft & kfSave) != 0) & (f.y >= g.twin0) & (f.y < g.twin1);
-
-        if (FULL && (ft & kfRf)) {
-            /* RF forward (src/mcx_core.cl:2833-2839): (w0 - w) / (mua + i omega n / c0) */
-            const float w0re = sh.pp[g.rfoff], w0im = sh.pp[g.rfoff + 1];
-            const float dre = w0re - rf.wre, dim = w0im - rf.wim;
-            const float aim = g.omega * s.prop.w * g.oneoverc0;
-            const float amag2 = s.prop.x * s.prop.x + aim * aim;
-            weight = (amag2 < K_EPS) ? (w0re * pathlen) : kdiv(dre * s.prop.x + dim * aim, amag2);
-            weight_im = (amag2 < K_EPS) ? (w0im * pathlen) : kdiv(dim * s.prop.x - dre * aim, amag2);
-        } else if (ft & kfFlux) {
-            float q = kdiv(s.w0 - p.w, s.prop.x);
-            K_PIN(q);
-            weight = (s.prop.x < K_EPS) ? (s.w0 * pathlen) : q;
-        } else if (g.outputtype == kEnergy) {
-            weight = s.w0 - p.w;
-        } else if (!SIMPLE && g.seed == K_SEED_FROM_FILE) {
-            if (deposits && (g.outputtype == kJacobian || (FULL && (g.outputtype == kRF || g.outputtype == kWLTOF)))) {
-                /* replay path deposits (src/mcx_core.cl:2845-2858): w L (J),
-                   -w L e^{i omega tof} (RF), tof w L (WLTOF) */
-                uint32_t pid = photon_index(g, idx, f.w) - 1;
-                weight = g.replayweight[pid] * pathlen;
-                tshift = gate_of(g, g.replaytof[pid]) +
-                         ((g.replaydet == -1) ? (((g.replaydetid[pid] & 0xFFFF) - 1) * (int)g.maxgate) : 0);
-
-                if (FULL && g.outputtype == kRF) {
-                    weight_im = -weight * sh.pp[g.w0offset + g.srcnum + 1];
-                    weight = -weight * sh.pp[g.w0offset + g.srcnum];
-                } else if (FULL && g.outputtype == kWLTOF) {
-                    weight = weight * g.replaytof[pid];
-                }
-            }
-        } else if (g.outputtype == kL) {
-            weight = s.w0 * pathlen;
-        }
-
-        if (!SIMPLE && (ft & kfSlots)) {
-            tshift += ((int)sh.pp[g.w0offset - 1] - 1) * ((g.replaydet == -1) ? (int)g.detnum : 1) *
-                      (int)g.maxgate;
-        }
-
-        deposits = deposits & (fabsf(weight) > 0.f);
-
-        if (FULL && (ft & kfPatterns)) {
-            if (deposits) {
-            /* several patterns share the photon: one interleaved slot per pattern
-               (src/mcx_core.cl:2902-2914), straight to the grid */
-            const uint32_t base = (oidx + (uint32_t)tshift * g.nvox) * g.npattern;
-
-            for (uint32_t i = 0; i < g.npattern; i++) {
-                const float pw = sh.pp[g.w0offset + i];
-
-                if (fabsf(pw) > 0.f) {
-                    deposit(g, sh.repoff, base + i, weight * pw);
-                }
-            }
-            }
-        } else {
-            const uint32_t dx = (uint32_t)(cx - (int)g.box_x0), dy = (uint32_t)(cy - (int)g.box_y0);
-            const uint32_t dz = (uint32_t)(cz - (int)g.box_z0);
-            const bool inbox = (dx < g.box_nx) & (dy < g.box_ny) & (dz < g.box_nz) & ((uint32_t)tshift < g.box_ng) &
-                               (lin0 == oidx);
-            gaddr = oidx + (uint32_t)tshift * g.nvox;
-
-            if (deposits & inbox) {
-                cell = sh.box + box_offset(g, (uint32_t)tshift, dx, dy, dz);
+                    if (deposits & inbox) {
+                        cell = sh.box + box_offset(g, (uint32_t)tshift, dx, dy, dz);
 #if MCX_PARITY
-                atomicAdd(cell, (BoxCell)weight);
+                        atomicAdd(cell, (BoxCell)weight);
 #else
-                boxold = atomicAdd(cell, weight);
-                boxval = weight;
+                        boxold = atomicAdd(cell, weight);
+                        boxval = weight;
 #endif
-            }
-
-            if (deposits & !inbox) {
-                evict = depcache_add(dcache, gaddr, weight, out_a, out_v);
-            }
-
-            /* a pattern source's deposit carries no imaginary term in the
-               reference (src/mcx_core.cl:2902-2914): its RF forward field
-               stays real */
-            if (FULL && (ft & kfRf) && deposits && g.srctype != kPattern && g.srctype != kPattern3D) {
-                deposit_voxel_im(g, sh, (lin0 == oidx) ? cx : -1, cy, cz, oidx, tshift, weight_im,
-                                 (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
-            }
-        }
-
-        if (FULL && (ft & kfRfReplay) && moved && f.y >= g.twin0 && f.y < g.twin1 && (ft & kfSave) &&
-                fabsf(weight_im) > 0.f) {
-            deposit(g, sh.repoff, oidx + (uint32_t)tshift * g.nvox + g.imoff, weight_im);
-        }
-
-        K_PIN(dcache.a0);
-        K_PIN(dcache.a1);
-        K_PIN(dcache.v0);
-        K_PIN(dcache.v1);
-        s.w0 = moved ? p.w : s.w0;
-        pathlen = moved ? 0.f : pathlen;
-
-        if (FULL && (ft & kfRf) && moved) {
-            sh.pp[g.rfoff] = rf.wre;
-            sh.pp[g.rfoff + 1] = rf.wim;
-        }
-
-        bool reflected = false;
-
-        /* the wait for the label belongs here, ahead of the grid atomic: the counter that
-           the wait uses also counts atomics, and this one then has until the next label
-           to complete */
-        K_PIN(lab);
-
-        if (evict) {
-            grid_add(g, sh.repoff + out_a, out_v);
-        }
-
-        s.mediaid = (cross & moved) ? (lab & K_MED_MASK) : s.mediaid;
-
-        if (SAVEDET) {
-            isdet = cross ? (lab & K_DET_MASK) : ((FULL && hitintf) ? detvox : (isdet | detvox));
-        } else {
-            isdet = 0;
-        }
-
-        if (FULL && (ft & kfSvmc)) {
-            /* split voxels (src/mcx_core.cl:2937-2949): a new voxel brings its own
-               plane and side; a plane crossing moves the photon to the other side */
-            if (cross) {
-                s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
-                testint = true;
-            } else if (hitintf) {
-                s.sn[0] = -s.sn[0];
-                s.sn[1] = -s.sn[1];
-                s.sn[2] = -s.sn[2];
-                s.sn[3] = -s.sn[3];
-                s.sv ^= 1u << 17;
-                testint = false;
-            }
-        }
-
-        /* split voxels also end the photon on entering label 0 through a voxel face
-           or the plane, unless it can reflect there (src/mcx_core.cl:2959-2966) */
-        const bool svexit = FULL && (ft & kfSvmc) && (cross || hitintf) && !K_SV_ISUPPER(s.sv) &&
-                            !K_SV_LOWER(s.sv) && (!g.doreflect || n1 == n0);
-        /* the index the photon comes from; the properties become the new voxel's (a
-           reflection reads the old ones again) */
-        const float nold = n1;
-
-        if (cross && !(FULL && (ft & kfSvmc))) {
-            s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
-        }
-
-        n1 = s.prop.w;
-#if !MCX_PARITY
-
-        box_move(g, sh, cell, boxold, boxval, gaddr, !SIMPLE && (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
-#endif
-        /* everything rare behind one test: a photon outside or in background, out of
-           time, of low weight, or at a change of index */
-        bool rare = (s.mediaid == 0) | svexit | !(f.y <= g.twin1) | (fabsf(p.w) < hold.minenergy);
-
-        if (REFLECT) {
-            rare = rare | (nold != n1) | (FULL && hitintf) | (FULL && (ft & kfMoveOnly));
-        }
-
-        if (!rare) {
-            if (SAVEDET) {
-                detvox = cross ? isdet : detvox;
-            }
-
-            continue;
-        }
-
-        if (cross & !in) {
-            isdet = ((s.idx1d == K_OUT_MAX ? bcmax : bcmin) >> (8 * face)) & 0xFFu;
-        }
-
-        const uint32_t code = isdet & 0xFu;
-        const bool mirror = code == kMirror;
-        const bool ends = ((s.mediaid == 0) & ((code == kAbsorb) | (code == kCyclic) | ((code == kReflect) & (nold == n0)))) |
-                          svexit | !(f.y <= g.twin1);
-
-        if (ends) {
-            bool wrapped = false;
-
-            if (isdet == kCyclic) {
-                if (face == 0) {
-                    p.x = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_x : 0.f), (v.x > 0.f) - (v.x < 0.f));
-                    s.fx = to_short((int)floorf(p.x));
-                }
-
-                if (face == 1) {
-                    p.y = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_y : 0.f), (v.y > 0.f) - (v.y < 0.f));
-                    s.fy = to_short((int)floorf(p.y));
-                }
-
-                if (face == 2) {
-                    p.z = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_z : 0.f), (v.z > 0.f) - (v.z < 0.f));
-                    s.fz = to_short((int)floorf(p.z));
-                }
-
-                if (inside(g, s.fx, s.fy, s.fz)) {
-                    s.idx1d = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
-                    s.mediaid = media_at(g, s.idx1d);
-                    isdet = s.mediaid & K_DET_MASK;
-                    detvox = isdet;
-                    s.mediaid &= K_MED_MASK;
-                    K_PIN(isdet);
-                    lin = s.idx1d;
-                    /* the next step still compares with the index of the voxel left here,
-                       as in the reference */
-                    n1 = nold;
-
-                    if (!(FULL && (ft & kfSvmc))) {
-                        s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
                     }
 
-                    wrapped = true;
+                    if (deposits & !inbox) {
+                        evict = depcache_add(dcache, gaddr, weight, out_a, out_v);
+                    }
+
+                    /* a pattern source's deposit carries no imaginary term in the
+                       reference (src/mcx_core.cl:2902-2914): its RF forward field
+                       stays real */
+                    if (FULL && (ft & kfRf) && deposits && g.srctype != kPattern && g.srctype != kPattern3D) {
+                        deposit_voxel_im(g, sh, (lin0 == oidx) ? cx : -1, cy, cz, oidx, tshift, weight_im,
+                                         (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
+                    }
                 }
-            }
 
-            if (!wrapped) {
-                launchflag = (((s.idx1d == K_OUT_MAX && ((bcdet >> (3 + face)) & 1u)) ||
-                               (s.idx1d == K_OUT_MIN && ((bcdet >> face) & 1u))) ? K_OUT_MIN : flag);
-                relaunch = true;
-                testint = testint || (FULL && (ft & kfSvmc));
-            }
-
-            continue;
-        }
-
-        if (fabsf(p.w) < g.minenergy) {
-            if (rng.next() * K_ROULETTE <= 1.f) {
-                p.w *= K_ROULETTE;
-
-                if (FULL && g.rfforward) {
-                    rf.wre *= K_ROULETTE;
-                    rf.wim *= K_ROULETTE;
-                    sh.pp[g.rfoff] *= K_ROULETTE;
-                    sh.pp[g.rfoff + 1] *= K_ROULETTE;
+                if (FULL && (ft & kfRfReplay) && moved && f.y >= g.twin0 && f.y < g.twin1 && (ft & kfSave) &&
+                        fabsf(weight_im) > 0.f) {
+                    deposit(g, sh.repoff, oidx + (uint32_t)tshift * g.nvox + g.imoff, weight_im);
                 }
-            } else {
-                launchflag = flag;
-                relaunch = true;
-                continue;
-            }
-        }
 
-        if (REFLECT) {
-            bool atface = true;
+                K_PIN(dcache.a0);
+                K_PIN(dcache.a1);
+                K_PIN(dcache.v0);
+                K_PIN(dcache.v1);
+                s.w0 = moved ? p.w : s.w0;
+                pathlen = moved ? 0.f : pathlen;
 
-            if (FULL && (ft & kfSvmc)) {
-                /* split voxels keep the properties of the side taken above; at the
-                   plane, Fresnel reflection or refraction between the two labels
-                   (src/mcx_core.cl:3072-3110) replaces the voxel-face test */
-                if (hitintf) {
-                    atface = false;
+                if (FULL && (ft & kfRf) && moved) {
+                    sh.pp[g.rfoff] = rf.wre;
+                    sh.pp[g.rfoff + 1] = rf.wim;
+                }
 
-                    if (sh.prop[K_SV_LOWER(s.sv)].w != sh.prop[K_SV_UPPER(s.sv)].w) {
+                bool reflected = false;
+
+                /* the wait for the label belongs here, ahead of the grid atomic: the counter that
+                   the wait uses also counts atomics, and this one then has until the next label
+                   to complete */
+                K_PIN(lab);
+
+                if (evict) {
+                    grid_add(g, sh.repoff + out_a, out_v);
+                }
+
+                s.mediaid = (cross & moved) ? (lab & K_MED_MASK) : s.mediaid;
+
+                if (SAVEDET) {
+                    isdet = cross ? (lab & K_DET_MASK) : ((FULL && hitintf) ? detvox : (isdet | detvox));
+                } else {
+                    isdet = 0;
+                }
+
+                if (FULL && (ft & kfSvmc)) {
+                    /* split voxels (src/mcx_core.cl:2937-2949): a new voxel brings its own
+                       plane and side; a plane crossing moves the photon to the other side */
+                    if (cross) {
+                        s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
+                        testint = true;
+                    } else if (hitintf) {
                         s.sn[0] = -s.sn[0];
                         s.sn[1] = -s.sn[1];
                         s.sn[2] = -s.sn[2];
                         s.sn[3] = -s.sn[3];
-
-                        if (svmc_reflect(nold, v, s, sh.prop, rng)) {
-                            launchflag = flag;
-                            relaunch = true;
-                            testint = true;
-                            continue;
-                        }
-                    } else {
-                        s.prop = sh.prop[K_SV_CURLABEL(s.sv)];
+                        s.sv ^= 1u << 17;
+                        testint = false;
                     }
                 }
-            }
 
-            const bool doref = (ft & kfReflect) != 0;
+                /* split voxels also end the photon on entering label 0 through a voxel face
+                   or the plane, unless it can reflect there (src/mcx_core.cl:2959-2966) */
+                const bool svexit = FULL && (ft & kfSvmc) && (cross || hitintf) && !K_SV_ISUPPER(s.sv) &&
+                                    !K_SV_LOWER(s.sv) && (!g.doreflect || n1 == n0);
+                /* the index the photon comes from; the properties become the new voxel's (a
+                   reflection reads the old ones again) */
+                const float nold = n1;
 
-            if (atface && (mirror | (nold != s.prop.w)) &&
-                    (s.mediaid ? doref : ((code == 0) & doref) | (code == kReflect) | mirror)) {
-                float Rtotal = 1.f;
-                float cphi, sphi, stheta, ctheta;
-                float tmp0 = nold * nold;
-                float tmp1 = s.prop.w * s.prop.w;
-                cphi = fabsf((face == 0) ? v.x : (face == 1 ? v.y : v.z));
-                sphi = 1.f - cphi * cphi;
-                f.z = 1.f - kdiv(tmp0, tmp1) * sphi;
-
-                if (f.z > 0.f && !mirror) {
-                    ctheta = tmp0 * cphi * cphi + tmp1 * f.z;
-                    stheta = 2.f * nold * s.prop.w * cphi * ksqrt(f.z);
-                    Rtotal = kdiv(ctheta - stheta, ctheta + stheta);
-                    ctheta = tmp1 * cphi * cphi + tmp0 * f.z;
-                    Rtotal = (Rtotal + kdiv(ctheta - stheta, ctheta + stheta)) * 0.5f;
+                if (cross && !(FULL && (ft & kfSvmc))) {
+                    s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
                 }
 
-                if (Rtotal < 1.f && (!(s.mediaid == 0 && mirror)) && rng.next() > Rtotal) {
-                    transmit(v, nold, s.prop.w, face);
+                n1 = s.prop.w;
+#if !MCX_PARITY
 
-                    if (s.mediaid == 0) {
+                box_move(g, sh, cell, boxold, boxval, gaddr,
+                         !SIMPLE && (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
+#endif
+                /* everything rare behind one test: a photon outside or in background, out of
+                   time, of low weight, or at a change of index */
+                bool rare = (s.mediaid == 0) | svexit | !(f.y <= g.twin1) | (fabsf(p.w) < hold.minenergy);
+
+                if (REFLECT) {
+                    rare = rare | (nold != n1) | (FULL && hitintf) | (FULL && (ft & kfMoveOnly));
+                }
+
+                if (!rare) {
+                    if (SAVEDET) {
+                        detvox = cross ? isdet : detvox;
+                    }
+
+                    continue;
+                }
+
+                if (cross & !in) {
+                    isdet = ((s.idx1d == K_OUT_MAX ? bcmax : bcmin) >> (8 * face)) & 0xFFu;
+                }
+
+                const uint32_t code = isdet & 0xFu;
+                const bool mirror = code == kMirror;
+                const bool ends = ((s.mediaid == 0) & ((code == kAbsorb) | (code == kCyclic) |
+                                                       ((code == kReflect) & (nold == n0)))) |
+                                  svexit | !(f.y <= g.twin1);
+
+                if (ends) {
+                    bool wrapped = false;
+
+                    if (isdet == kCyclic) {
+                        if (face == 0) {
+                            p.x = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_x : 0.f),
+                                                (v.x > 0.f) - (v.x < 0.f));
+                            s.fx = to_short((int)floorf(p.x));
+                        }
+
+                        if (face == 1) {
+                            p.y = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_y : 0.f),
+                                                (v.y > 0.f) - (v.y < 0.f));
+                            s.fy = to_short((int)floorf(p.y));
+                        }
+
+                        if (face == 2) {
+                            p.z = nextafter_ref(rintf((s.idx1d == K_OUT_MIN) ? g.maxidx_z : 0.f),
+                                                (v.z > 0.f) - (v.z < 0.f));
+                            s.fz = to_short((int)floorf(p.z));
+                        }
+
+                        if (inside(g, s.fx, s.fy, s.fz)) {
+                            s.idx1d = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+                            s.mediaid = media_at(g, s.idx1d);
+                            isdet = s.mediaid & K_DET_MASK;
+                            detvox = isdet;
+                            s.mediaid &= K_MED_MASK;
+                            K_PIN(isdet);
+                            lin = s.idx1d;
+                            /* the next step still compares with the index of the voxel left here,
+                               as in the reference */
+                            n1 = nold;
+
+                            if (!(FULL && (ft & kfSvmc))) {
+                                s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
+                            }
+
+                            wrapped = true;
+                        }
+                    }
+
+                    if (!wrapped) {
                         launchflag = (((s.idx1d == K_OUT_MAX && ((bcdet >> (3 + face)) & 1u)) ||
                                        (s.idx1d == K_OUT_MIN && ((bcdet >> face) & 1u))) ? K_OUT_MIN : flag);
                         relaunch = true;
+                        testint = testint || (FULL && (ft & kfSvmc));
+                    }
+
+                    continue;
+                }
+
+                if (fabsf(p.w) < g.minenergy) {
+                    if (rng.next() * K_ROULETTE <= 1.f) {
+                        p.w *= K_ROULETTE;
+
+                        if (FULL && g.rfforward) {
+                            rf.wre *= K_ROULETTE;
+                            rf.wim *= K_ROULETTE;
+                            sh.pp[g.rfoff] *= K_ROULETTE;
+                            sh.pp[g.rfoff + 1] *= K_ROULETTE;
+                        }
+                    } else {
+                        launchflag = flag;
+                        relaunch = true;
                         continue;
                     }
-                } else {
-                    if (face == 0) {
-                        v.x = -v.x;
-                        p.x = nextafter_ref(rintf(p.x), 0);
-                        s.fx = to_short((int)rintf(p.x));
-                    } else if (face == 1) {
-                        v.y = -v.y;
-                        p.y = nextafter_ref(rintf(p.y), 0);
-                        s.fy = to_short((int)rintf(p.y));
-                    } else {
-                        v.z = -v.z;
-                        p.z = nextafter_ref(rintf(p.z), 0);
-                        s.fz = to_short((int)rintf(p.z));
-                    }
+                }
 
-                    /* back in the voxel it came from, with its label and properties */
-                    s.idx1d = oidx;
-                    s.mediaid = omed;
-                    reflected = true;
-                    lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+                if (REFLECT) {
+                    bool atface = true;
 
-                    if (!(FULL && (ft & kfSvmc))) {
-                        s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
-                    } else {
-                        /* the side of the plane the reflected photon lands on; label 0
-                           there ends it (src/mcx_core.cl:3221-3243) */
-                        s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
+                    if (FULL && (ft & kfSvmc)) {
+                        /* split voxels keep the properties of the side taken above; at the
+                           plane, Fresnel reflection or refraction between the two labels
+                           (src/mcx_core.cl:3072-3110) replaces the voxel-face test */
+                        if (hitintf) {
+                            atface = false;
 
-                        if (K_SV_CURLABEL(s.sv) == 0) {
-                            launchflag = flag;
-                            relaunch = true;
-                            continue;
+                            if (sh.prop[K_SV_LOWER(s.sv)].w != sh.prop[K_SV_UPPER(s.sv)].w) {
+                                s.sn[0] = -s.sn[0];
+                                s.sn[1] = -s.sn[1];
+                                s.sn[2] = -s.sn[2];
+                                s.sn[3] = -s.sn[3];
+
+                                if (svmc_reflect(nold, v, s, sh.prop, rng)) {
+                                    launchflag = flag;
+                                    relaunch = true;
+                                    testint = true;
+                                    continue;
+                                }
+                            } else {
+                                s.prop = sh.prop[K_SV_CURLABEL(s.sv)];
+                            }
                         }
                     }
 
-                    /* drop the boundary code so a later same-voxel step restores
-                       the voxel's own label (the reference ORs the code in) */
-                    isdet &= K_DET_MASK;
+                    const bool doref = (ft & kfReflect) != 0;
+
+                    if (atface && (mirror | (nold != s.prop.w)) &&
+                            (s.mediaid ? doref : ((code == 0) & doref) | (code == kReflect) | mirror)) {
+                        float Rtotal = 1.f;
+                        float cphi, sphi, stheta, ctheta;
+                        float tmp0 = nold * nold;
+                        float tmp1 = s.prop.w * s.prop.w;
+                        cphi = fabsf((face == 0) ? v.x : (face == 1 ? v.y : v.z));
+                        sphi = 1.f - cphi * cphi;
+                        f.z = 1.f - kdiv(tmp0, tmp1) * sphi;
+
+                        if (f.z > 0.f && !mirror) {
+                            ctheta = tmp0 * cphi * cphi + tmp1 * f.z;
+                            stheta = 2.f * nold * s.prop.w * cphi * ksqrt(f.z);
+                            Rtotal = kdiv(ctheta - stheta, ctheta + stheta);
+                            ctheta = tmp1 * cphi * cphi + tmp0 * f.z;
+                            Rtotal = (Rtotal + kdiv(ctheta - stheta, ctheta + stheta)) * 0.5f;
+                        }
+
+                        if (Rtotal < 1.f && (!(s.mediaid == 0 && mirror)) && rng.next() > Rtotal) {
+                            transmit(v, nold, s.prop.w, face);
+
+                            if (s.mediaid == 0) {
+                                launchflag = (((s.idx1d == K_OUT_MAX && ((bcdet >> (3 + face)) & 1u)) ||
+                                               (s.idx1d == K_OUT_MIN && ((bcdet >> face) & 1u))) ? K_OUT_MIN : flag);
+                                relaunch = true;
+                                continue;
+                            }
+                        } else {
+                            if (face == 0) {
+                                v.x = -v.x;
+                                p.x = nextafter_ref(rintf(p.x), 0);
+                                s.fx = to_short((int)rintf(p.x));
+                            } else if (face == 1) {
+                                v.y = -v.y;
+                                p.y = nextafter_ref(rintf(p.y), 0);
+                                s.fy = to_short((int)rintf(p.y));
+                            } else {
+                                v.z = -v.z;
+                                p.z = nextafter_ref(rintf(p.z), 0);
+                                s.fz = to_short((int)rintf(p.z));
+                            }
+
+                            /* back in the voxel it came from, with its label and properties */
+                            s.idx1d = oidx;
+                            s.mediaid = omed;
+                            reflected = true;
+                            lin = (uint32_t)(s.fz * (int)g.dimxy + s.fy * (int)g.dimx + s.fx);
+
+                            if (!(FULL && (ft & kfSvmc))) {
+                                s.prop = getprop<FULL, true>(g, sh, s.mediaid, s.idx1d, ft);
+                            } else {
+                                /* the side of the plane the reflected photon lands on; label 0
+                                   there ends it (src/mcx_core.cl:3221-3243) */
+                                s.prop = svmc_prop(g, sh.prop, s.mediaid, s.idx1d, p, s.fx, s.fy, s.fz, s);
+
+                                if (K_SV_CURLABEL(s.sv) == 0) {
+                                    launchflag = flag;
+                                    relaunch = true;
+                                    continue;
+                                }
+                            }
+
+                            /* drop the boundary code so a later same-voxel step restores
+                               the voxel's own label (the reference ORs the code in) */
+                            isdet &= K_DET_MASK;
+                        }
+                    }
+
+                    if (FULL && (ft & kfMoveOnly) && (s.mediaid == 0 || s.idx1d == K_OUT_MIN || s.idx1d == K_OUT_MAX)) {
+                        /* move-only trajectories (debug flag T, src/mcx_core.cl:3287-3291): the
+                           lane's whole run ends here, without its energy write-back */
+                        break;
+                    }
                 }
-            }
 
-            if (FULL && (ft & kfMoveOnly) && (s.mediaid == 0 || s.idx1d == K_OUT_MIN || s.idx1d == K_OUT_MAX)) {
-                /* move-only trajectories (debug flag T, src/mcx_core.cl:3287-3291): the
-                   lane's whole run ends here, without its energy write-back */
-                break;
-            }
+                n1 = s.prop.w;
+
+                if (SAVEDET) {
+                    detvox = (cross & !reflected) ? (isdet & K_DET_MASK) : detvox;
+                }
+            }   /* the step loop */
         }
 
-        n1 = s.prop.w;
-
-        if (SAVEDET) {
-            detvox = (cross & !reflected) ? (isdet & K_DET_MASK) : detvox;
+        if (thresh == 0) {
+            break;
         }
-    }
-    }
 
-    if (thresh == 0) {
-        break;
-    }
-
-    alive = hand_over(sh, put, rng, from);
-    moved_on = true;
-    thresh = 0;
-    asm("" : "+s"(thresh));   /* one copy of the step loop for both */
+        alive = hand_over(sh, put, rng, from);
+        moved_on = true;
+        thresh = 0;
+        asm("" : "+s"(thresh));   /* one copy of the step loop for both */
     }
 
     depcache_flush(g, sh, dcache);
