@@ -13,10 +13,10 @@
    launches 256-lane workgroups.  The fast build runs one workgroup per CU, so
    that a single LDS deposit box can use most of the CU's LDS instead of being
    split between several workgroups: 1024 lanes (16 waves, <=128 VGPRs) for the
-   pencil-beam specialisation (101 VGPRs) and for the general path without
+   pencil-beam specialisation (97-100 VGPRs) and for the general path without
    detected photons or without reflection (11-13 VGPRs spilled to scratch outside
    the step loop, 6-9% faster than 768 lanes), 768 lanes (12 waves, <=168 VGPRs, no
-   spills) for the general path with both (152 VGPRs). */
+   spills) for the general path with both (154 VGPRs). */
 #define MCX_MAX_BLOCK 256
 /* a wave hands its lanes over once at most this many are live (a quarter: the lanes of
    four waves fit in one), and the words a lane moves besides its LDS scratch */
@@ -26,7 +26,8 @@
 #define MCX_BOX_LIMIT 256.f
 #define MCX_BOX_LIMIT_MIN 32.f
 #define MCX_FAST_SIMPLE_BLOCK 1024
-/* waves per SIMD the fast kernels are built for (amdgpu_waves_per_eu caps them) */
+/* waves per SIMD of the fast kernels: the transport kernels are built for no more
+   (amdgpu_waves_per_eu), the batched kernel's 128 VGPRs leave room for no more */
 #define MCX_FAST_WAVES 4
 #define MCX_FAST_BLOCK 1024
 #define MCX_FAST_DETREF_BLOCK 768

@@ -38,9 +38,9 @@ extern "C" hipError_t mcx_launch_fast(const MCXKParam* prm, int nblock, int nthr
 
 /* Resident workgroups per CU of a kernel from its own register and LDS use and
    gfx950's per-CU resources: 4 SIMDs, each holding at most MCX_FAST_WAVES waves
-   (the kernels' own cap; the hardware's is 8) and 512 VGPRs per lane allocated in
-   granules of 8, and the device's LDS per CU in
-   512-byte granules per workgroup.  A workgroup spreads its waves over the 4
+   (what these kernels are built for or have registers for; the hardware's limit is
+   8) and 512 VGPRs per lane allocated in granules of 8, and the device's LDS per CU
+   in 512-byte granules per workgroup.  A workgroup spreads its waves over the 4
    SIMDs.  (The runtime's occupancy query has returned half of this count on
    some MI355X hosts for the same code object, ruling out 1024-lane workgroups
    that launch and run there.) */

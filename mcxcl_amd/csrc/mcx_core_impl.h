@@ -18,7 +18,8 @@
  *    here every termination sets a flag and the loop head relaunches, so the
  *    large launch body is emitted once and lanes reconverge there;
  *  - the medium table and the phase-function inverse CDF are staged in LDS;
- *    the per-lane partial-path/energy scratch lives in LDS (wave64 stride);
+ *    the per-lane record scratch (partial paths, source id, pattern weights)
+    lives in LDS (wave64 stride); a lane's energies are registers;
  *  - fluence is accumulated with native global_atomic_add_f64 into a double
  *    grid (no MAX_ACCUM shadow half is needed), converted and normalised by a
  *    separate streaming kernel;
@@ -354,7 +355,7 @@ struct Shared {
     float4* prop;                /* medium table */
     float* invcdf;
     BoxCell* box;                /* privatised deposit box (box_cells) */
-    float* pp;                   /* this lane's scratch: partial data, energies, w0, srcid */
+    float* pp;                   /* this lane's scratch: partial data, w0, srcid, ... (pplen floats) */
     size_t repoff;               /* offset of this workgroup's global accumulator replica */
     uint32_t* wlive;             /* live lanes per wave, for the hand-over (LDS) */
     uint32_t* hand;              /* this workgroup's hand-over slots (global memory): word k of slot j at
@@ -1825,15 +1826,15 @@ __device__ __forceinline__ bool hand_over(const Shared& sh, bool put, Rng& rng, 
    waves merge (hand_over).  A load still in flight where branches meet makes the
    compiler wait for all of them at the head of the loop, the grid atomics too, so
    every load is pinned where it is read.
-   Measured (MI355X, kernel time): the loop that reloaded label and properties at every
-   step, this loop, this loop with the hand-over and the pinned loads:
-     packed media, isotropic source, 71x64x53, 3e6 photons     169, 113, 111 ms
-     layered 200^3, pencil beam, 1e7 photons                   151, 122, 116 ms
-     60^3 cube, pencil beam, 3e5 photons                       7.2, 6.0, 4.5 ms
-     60^3 sphere, 2e4 photons with records, parity arithmetic  18.0, 16.2, 12.1 ms
-     four 96^3 sources and detectors, parity arithmetic        82, 66, 61 ms
-     batch of 16 48^3 instances                                867, 764, 740 ms
-     60^3 sphere, pencil beam, 1e8 photons (grid atomics)      423, 420, 420 ms */
+   Measured (MI355X, kernel time, in turn on one card): the loop that reloaded label and
+   properties at every step, its waves run to their end, and this loop:
+     packed media, isotropic source, 71x64x53, 3e6 photons     181, 119 ms
+     layered 200^3, pencil beam, 1e7 photons                   150, 115 ms
+     60^3 cube, pencil beam, 3e5 photons                       7.3, 4.6 ms
+     60^3 sphere, 2e4 photons with records, parity arithmetic  17.3, 12.1 ms
+     four 96^3 sources and detectors, parity arithmetic        81, 61 ms
+     batch of 16 48^3 instances, three draws of them           873, 800; 1009, 889; 863, 756 ms
+     60^3 sphere, pencil beam, 1e8 photons (grid atomics)      419, 408 ms */
 /* Transport this lane's photons until its share (fixed map) or its
    workgroup's pool (run-time hand-out) is exhausted.  The photon state starts
    fresh; the RNG, the LDS tables and the lane's scratch come in, and the

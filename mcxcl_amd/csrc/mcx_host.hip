@@ -683,7 +683,7 @@ size_t mcx_kparam_setup(Config* cfg, MCXKParam* gp, size_t nthread, size_t lbloc
        nearly all of its deposits, so there the limit is the lower one.  Error of the
        fluence against float64 sums (2-norm) with the box at the source's corner and moves
        at 1024, and under it with limits 256 and 32:
-         40x40 on 60^3, 1e7 photons                1.2e-8, 1.9e-8, 8.7e-9 (38.1, 38.2 ms)
+         40x40 on 60^3, 1e7 photons                1.2e-8, 1.9e-8, 8.7e-9 (37.9, 38.6 ms)
          20x53 on 31x80x40, 6 gates, 1.2e7 photons 2.9e-8, 6.7e-8, 9.0e-9 */
     g.box_tight = fmaxf(width[0], 1.f) * fmaxf(width[1], 1.f) * fmaxf(width[2], 1.f) >= 8.f;
 
