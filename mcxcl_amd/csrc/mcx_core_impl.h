@@ -432,12 +432,13 @@ __device__ __forceinline__ uint32_t box_offset(const MCXKParam& g, uint32_t gate
     return mad24(mad24(mad24(gate, g.box_nz, dz), g.box_ny, dy), g.box_nx, dx);
 }
 
-/* the move that a deposit of val brings about in a cell that held old: idx the cell's
-   place in the replica of the grid */
+/* the move that a deposit of val brings about in a cell that held old (NaN: there was no
+   deposit): idx the cell's place in the replica of the grid */
 __device__ __forceinline__ void box_move(const MCXKParam& g, const Shared& sh, BoxCell* cell, float old, float val,
         uint32_t idx, float limit) {
     const float now = old + val;    /* the cell's own sum: both round to nearest */
 
+    /* old too: a deposit of the other sign may cross back while an excess is under way */
     if (fmaxf(fabsf(old), fabsf(now)) >= limit) {
         /* a power of two: its reciprocal and the products with it are exact */
         const float twice = 2.f * limit, inv = 1.f / twice;
@@ -2313,7 +2314,7 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
                 const bool moved = (cross | (FULL && hitintf)) & (oidx < g.nvox) & ((omed | isdet) != 0);
                 const uint32_t flag = isdet;
                 BoxCell* cell = sh.box;
-                float boxold = 0.f, boxval = 0.f;
+                float boxold = __uint_as_float(0x7FC00000u);
                 uint32_t gaddr = 0, out_a = 0;
                 double out_v = 0.0;
                 bool evict = false;
@@ -2399,7 +2400,6 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
                         atomicAdd(cell, (BoxCell)weight);
 #else
                         boxold = atomicAdd(cell, weight);
-                        boxval = weight;
 #endif
                     }
 
@@ -2483,7 +2483,7 @@ __device__ __forceinline__ void transport_lane(const MCXKParam& g, const Shared&
                 n1 = s.prop.w;
 #if !MCX_PARITY
 
-                box_move(g, sh, cell, boxold, boxval, gaddr,
+                box_move(g, sh, cell, boxold, weight, gaddr,
                          !SIMPLE && (ft & kfTight) ? MCX_BOX_LIMIT_MIN : MCX_BOX_LIMIT);
 #endif
                 /* everything rare behind one test: a photon outside or in background, out of
