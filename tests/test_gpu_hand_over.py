@@ -159,6 +159,23 @@ def test_replays_move_whole(recorded, outputtype, replaydet, monkeypatch):
     _agree(mcxcl_amd.run(cfg), ref, _keys(cfg))
 
 
+@pytest.mark.parametrize("outputtype", ["jacobian", "wp", "wm", "rf", "rfmus", "wltof", "wptof"])
+def test_fast_replays_move_whole(recorded, outputtype, monkeypatch):
+    """the default arithmetic's replay on a fixed map, in 256-lane workgroups and in the spread
+    that moves nothing: the same photons, so the grids differ by the float32 box's rounding
+    alone (below 1e-6 of the whole)"""
+    base, _ = recorded
+    fwd = mcxcl_amd.run(dict(base, mathmode=0))
+    assert fwd["detp"].shape[1] > 300
+    cfg = dict(base, seed=fwd["seeds"], detphotons=fwd["detp"], replayweight=fwd["detw"], outputtype=outputtype,
+               replaydet=0, omega=_OMEGA, savedetweight=0, mathmode=0, rawfield=1, rawonly=1)
+    spread = mcxcl_amd.run(cfg)["flux64"]
+    monkeypatch.setenv("MCXHIP_BLOCK", "256")
+    moved = mcxcl_amd.run(cfg)["flux64"]
+    size, err = np.linalg.norm(spread), np.linalg.norm(moved - spread)
+    assert size > 0 and err <= 1e-6 * size
+
+
 def _absorbed(out, n):
     """absorbed and deposited weight per photon"""
     return np.array([out["stat"]["energyabs"], out["flux64"].sum()]) / n
